@@ -49,6 +49,7 @@ void launch_chunk_prefill_any(bool, const ChunkAttnParams&, hipStream_t);
 void launch_chunk_decode(bool, const ChunkAttnParams&, hipStream_t);
 
 void launch_stream_gemm(const StreamGemmParams&, int, hipStream_t);
+int stream_gemm_partials(const StreamGemmParams&, int);  // partial sums of squares per row
 
 namespace {
 
@@ -208,15 +209,15 @@ at::Tensor relu2(const at::Tensor& u_) {
   return y;
 }
 
-// Decode projections, <= 32 rows (stream_gemm.hip)
+// Decode projections, <= 64 rows (stream_gemm.hip)
 StreamGemmParams gemm_params(const at::Tensor& a, const at::Tensor& w, int64_t per_col, const OptT& ssq_in, double eps) {
   check_bf16(a, "a");
   check_bf16(w, "w");
   same_device(a, w);
   TORCH_CHECK(a.dim() == 2 && a.is_contiguous() && w.dim() == 2 && w.is_contiguous() && a.size(1) == w.size(1), "a [M, K], w [N, K]");
   const int64_t M = a.size(0), N = w.size(0) / per_col, K = w.size(1);
-  TORCH_CHECK(M >= 1 && M <= 32 && N >= 1 && N < (1 << 24) && w.size(0) == N * per_col && K >= 8 && K < (1 << 24) && K % 8 == 0,
-              "stream_gemm: 1 <= M <= 32, K % 8 == 0");
+  TORCH_CHECK(M >= 1 && M <= 64 && N >= 1 && N < (1 << 24) && w.size(0) == N * per_col && K >= 8 && K < (1 << 24) && K % 8 == 0,
+              "stream_gemm: 1 <= M <= 64, K % 8 == 0");
   check_aligned16(a, "a");
   check_aligned16(w, "w");
   StreamGemmParams p{};
@@ -236,7 +237,7 @@ StreamGemmParams gemm_params(const at::Tensor& a, const at::Tensor& w, int64_t p
 }
 
 // the fp32 stream and the partial sums of squares of an epilogue that updates it; returns ssq
-at::Tensor gemm_stream(StreamGemmParams& p, const at::Tensor& a, const at::Tensor& x, const OptT& norm_w) {
+at::Tensor gemm_stream(StreamGemmParams& p, int epi, const at::Tensor& a, const at::Tensor& x, const OptT& norm_w) {
   check_f32(x, "x");
   TORCH_CHECK(x.numel() == static_cast<int64_t>(p.M) * p.N && x.size(-1) == p.N && x.is_contiguous() && x.device() == a.device(), "x [M, N]");
   p.x = x.data_ptr<float>();
@@ -244,7 +245,7 @@ at::Tensor gemm_stream(StreamGemmParams& p, const at::Tensor& a, const at::Tenso
     vec_like(*norm_w, a, p.N, "norm_w");
     p.norm_w = cbp(*norm_w);
   }
-  auto ssq = at::empty({p.M, (p.N + 15) / 16}, x.options());
+  auto ssq = at::empty({p.M, stream_gemm_partials(p, epi)}, x.options());
   p.ssq = ssq.data_ptr<float>();
   return ssq;
 }
@@ -262,7 +263,7 @@ std::tuple<at::Tensor, at::Tensor> stream_gemm(const at::Tensor& a, const at::Te
   at::Tensor ssq;
   if (epi == 3) {
     TORCH_CHECK(x.has_value(), "stream epilogue: x");
-    ssq = gemm_stream(p, a, *x, norm_w);
+    ssq = gemm_stream(p, 3, a, *x, norm_w);
   } else {
     ssq = at::empty({0}, a.options().dtype(at::kFloat));
   }
@@ -289,7 +290,7 @@ std::tuple<at::Tensor, at::Tensor> stream_gemm_post(const at::Tensor& a, const a
   c10::hip::HIPGuardMasqueradingAsCUDA guard(a.device());
   auto y = at::empty({p.M, p.N}, a.options());
   p.y = bp(y);
-  at::Tensor ssq = gemm_stream(p, a, x, norm_w);
+  at::Tensor ssq = gemm_stream(p, 4, a, x, norm_w);
   p.alpha = static_cast<float>(alpha);
   if (bias.has_value()) {
     vec_like(*bias, a, p.N, "bias");

@@ -136,7 +136,7 @@ struct StreamGemmParams {
   float* x;                // stream epilogue: fp32 [M, N], updated in place
   const uint16_t* norm_w;  // stream epilogue: the next norm's weight, or nullptr
   float offset;
-  float* ssq;              // stream epilogue: [M, ceil(N / 16)]
+  float* ssq;              // stream epilogue: [M, stream_gemm_partials]
   float alpha;             // post epilogue: x <- alpha x_prev + . + bias
   const float* res_ssq;    // post epilogue: x holds a sum before its norm; [M, nres] partial sums of squares, or nullptr
   int nres;
@@ -147,6 +147,7 @@ struct StreamGemmParams {
   const int64_t* ids;      // gate epilogue: [M]
   const uint16_t* table;
   int64_t ldt, off, vocab;
+  int nt;                  // weights by non-temporal loads (set by the launcher)
 };
 
 }  // namespace dla

@@ -117,15 +117,15 @@ def head_logits(h: torch.Tensor, w: torch.Tensor, cap: float = 0.0) -> torch.Ten
 # (csrc/mix/stream_gemm.hip) few rows: the norm before a projection and the stream add / activation /
 # gate behind it run inside the projection's launch. DLA_STREAM_FUSED=0: library GEMMs + the kernels above.
 STREAM_FUSED = os.environ.get("DLA_STREAM_FUSED", "1") != "0"
-# (17 .. 32 rows run too, but every workgroup re-reads all of a for its 16 columns: at 32 rows that is
-# more L2 traffic than the weights, and the library's GEMMs are ahead)
-STREAM_FUSED_ROWS = int(os.environ.get("DLA_STREAM_FUSED_ROWS", "16"))
+# (up to 64 rows, what the kernel takes: the library's GEMM of 2048 x 8192 alone takes 15.6 us at 32 rows, the fused
+# form with its sum and the next norm's partials 14.2; of 128 x 2048 10.6 against 4.1 with the gate)
+STREAM_FUSED_ROWS = int(os.environ.get("DLA_STREAM_FUSED_ROWS", "64"))
 _STORE, _RELU2, _GATE, _STREAM, _GEGLU = 0, 1, 2, 3, 5  # (4, 6: ops of their own)
 
 
 def fused_ok(rows: int, dtype: torch.dtype, *weights: torch.Tensor) -> bool:
-    """These projections can run on the fused decode kernel (bf16, GPU, <= 32 rows, K % 8 == 0)."""
-    return (STREAM_FUSED and 1 <= rows <= min(STREAM_FUSED_ROWS, 32) and dtype == torch.bfloat16
+    """These projections can run on the fused decode kernel (bf16, GPU, <= 64 rows, K % 8 == 0)."""
+    return (STREAM_FUSED and 1 <= rows <= min(STREAM_FUSED_ROWS, 64) and dtype == torch.bfloat16
             and all(w.is_cuda and w.dim() == 2 and w.is_contiguous() and w.shape[1] % 8 == 0 and w.data_ptr() % 16 == 0
                     for w in weights))
 
