@@ -856,7 +856,8 @@ at::Tensor latent_decode(const at::Tensor& q, const at::Tensor& latent, const at
   ns = std::min<int64_t>(ns, (most + tile - 1) / tile);
   p.ns = static_cast<int>(std::max<int64_t>(1, std::min<int64_t>(ns, 256)));
   c10::hip::HIPGuardMasqueradingAsCUDA guard(q.device());
-  auto qcat = at::empty({p.B, H, p.R + rot}, q.options());
+  // (whole groups of 16 heads, and 576 columns for what is padded to 18 steps of 32)
+  auto qcat = at::empty({p.B, (H + 15) / 16 * 16, std::max<int64_t>(576, p.R + rot)}, q.options());
   auto po = at::empty({p.B, H, p.ns, p.R}, q.options().dtype(at::kFloat));
   auto ml = at::empty({p.B, H, p.ns, 2}, po.options());
   auto o = at::empty({p.B, 1, H * vdim}, q.options());

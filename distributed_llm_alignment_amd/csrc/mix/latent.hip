@@ -14,10 +14,12 @@
 // weights (hi + lo planes on bf16 MFMAs) and all sums are fp32.
 #include "mix_params.h"
 #include "mma.h"
+#include "state_step.h"
 
 namespace dla {
 
 bool latent_decode_mfma_ok(const LatentParams&);  // latent_decode.hip
+int latent_decode_mfma_steps(const LatentParams&);  // 32-wide steps over a query's columns
 void launch_latent_decode_mfma(const LatentParams&, hipStream_t);
 
 namespace {
@@ -43,44 +45,77 @@ __global__ __launch_bounds__(128) void latent_prepare_kernel(
     T* __restrict__ cq, T* __restrict__ latent, int64_t l_sb, int64_t l_st, const int64_t* __restrict__ slot,
     const int* __restrict__ kv_start, const float* __restrict__ cos_t, const float* __restrict__ sin_t, int Tn,
     int qr, int R, int rot, int tcap) {
-  __shared__ float scratch[2];
+  __shared__ float scratch[4];
   const int64_t row = blockIdx.x;
   const int b = static_cast<int>(row / Tn), t = static_cast<int>(row % Tn);
   const int64_t col = min(slot[0] + t, static_cast<int64_t>(tcap - 1));  // (a full cache is the host's error)
   const T* in = down + row * ld;
   T* out = latent + b * l_sb + col * l_st;
-  float sq = 0.f, sk = 0.f, v[VEC], w[VEC];
-  for (int i = threadIdx.x * VEC; i < qr; i += 128 * VEC) {
+  // a thread's first piece of both rows, of both weights and of the rotated part are loaded side by side and stay in
+  // registers (a row of up to 128 VEC is one piece)
+  const int i0 = threadIdx.x * VEC, step = 128 * VEC;
+  float q0[VEC], k0[VEC], wq[VEC], wk[VEC], v[VEC], w[VEC];
+#pragma unroll
+  for (int e = 0; e < VEC; ++e) q0[e] = k0[e] = wq[e] = wk[e] = 0.f;
+  if (i0 < qr) {
+    load_vec<T, VEC>(in + i0, q0);
+    load_vec<T, VEC>(qw + i0, wq);
+  }
+  if (i0 < R) {
+    load_vec<T, VEC>(in + qr + i0, k0);
+    load_vec<T, VEC>(kw + i0, wk);
+  }
+  const int64_t pos = max(col - (kv_start ? kv_start[b] : 0), static_cast<int64_t>(0));
+  const float *cs = cos_t + pos * (rot >> 1), *sn = sin_t + pos * (rot >> 1);
+  float rv = 0.f;
+  const int ri = threadIdx.x;
+  if (ri < rot) load_rotated<T, 1>(in + qr + R, ri, rot, cs, sn, &rv);
+  float sq = 0.f, sk = 0.f;
+#pragma unroll
+  for (int e = 0; e < VEC; ++e) {
+    sq += q0[e] * q0[e];
+    sk += k0[e] * k0[e];
+  }
+  for (int i = i0 + step; i < qr; i += step) {
     load_vec<T, VEC>(in + i, v);
 #pragma unroll
     for (int e = 0; e < VEC; ++e) sq += v[e] * v[e];
   }
-  for (int i = threadIdx.x * VEC; i < R; i += 128 * VEC) {
+  for (int i = i0 + step; i < R; i += step) {
     load_vec<T, VEC>(in + qr + i, v);
 #pragma unroll
     for (int e = 0; e < VEC; ++e) sk += v[e] * v[e];
   }
-  const float rq = rsqrtf(block_sum<128>(sq, scratch) / qr + eps);
-  const float rk = rsqrtf(block_sum<128>(sk, scratch) / R + eps);
-  for (int i = threadIdx.x * VEC; i < qr; i += 128 * VEC) {
+  sq = wave_sum(sq);
+  sk = wave_sum(sk);
+  if ((threadIdx.x & 63) == 0) {
+    scratch[threadIdx.x >> 6] = sq;
+    scratch[2 + (threadIdx.x >> 6)] = sk;
+  }
+  __syncthreads();
+  const float rq = rsqrtf((scratch[0] + scratch[1]) / qr + eps), rk = rsqrtf((scratch[2] + scratch[3]) / R + eps);
+  auto scaled = [&](const float* x, const float* y, float f, T* to) {
+    float o[VEC];
+#pragma unroll
+    for (int e = 0; e < VEC; ++e) o[e] = x[e] * f * y[e];
+    store_vec<T, VEC>(to, o);
+  };
+  if (i0 < qr) scaled(q0, wq, rq, cq + row * qr + i0);
+  if (i0 < R) scaled(k0, wk, rk, out + i0);
+  for (int i = i0 + step; i < qr; i += step) {
     load_vec<T, VEC>(in + i, v);
     load_vec<T, VEC>(qw + i, w);
-#pragma unroll
-    for (int e = 0; e < VEC; ++e) v[e] = v[e] * rq * w[e];
-    store_vec<T, VEC>(cq + row * qr + i, v);
+    scaled(v, w, rq, cq + row * qr + i);
   }
-  for (int i = threadIdx.x * VEC; i < R; i += 128 * VEC) {
+  for (int i = i0 + step; i < R; i += step) {
     load_vec<T, VEC>(in + qr + i, v);
     load_vec<T, VEC>(kw + i, w);
-#pragma unroll
-    for (int e = 0; e < VEC; ++e) v[e] = v[e] * rk * w[e];
-    store_vec<T, VEC>(out + i, v);
+    scaled(v, w, rk, out + i);
   }
-  const int64_t pos = max(col - (kv_start ? kv_start[b] : 0), static_cast<int64_t>(0));
-  for (int i = threadIdx.x; i < rot; i += 128) {
-    float r;
-    load_rotated<T, 1>(in + qr + R, i, rot, cos_t + pos * (rot >> 1), sin_t + pos * (rot >> 1), &r);
-    out[R + i] = from_f<T>(r);
+  if (ri < rot) out[R + ri] = from_f<T>(rv);
+  for (int i = ri + 128; i < rot; i += 128) {
+    load_rotated<T, 1>(in + qr + R, i, rot, cs, sn, &rv);
+    out[R + i] = from_f<T>(rv);
   }
 }
 
@@ -223,18 +258,45 @@ int prefill_waves(const LatentParams& p) {
 }
 
 // ------------------------------------------------------------------------------------- absorb
-// qcat[b][h] = [sum_d q[b][h][d] W_uk[h][d][:] | rotated q part]. grid (H, ceil(R / 64)), 256 threads:
-// 8 column groups of 8 x 32 slices of d; batch rows in groups of 4.
+// qcat[b][h] = [sum_d q[b][h][d] W_uk[h][d][:] | rotated q part]. grid (H, ceil(R / 64) + 1), 256 threads:
+// 8 column groups of 8 x 32 slices of d; batch rows in groups of 4. The last row of blocks rotates.
+//
+// Column c of a query in latent space: rows [B, H, R + rot], or, with `qsteps`, in the order in which the MFMA decode
+// kernel's lanes hold it (k-step, lane, 8 columns): one of its loads is then 1 KB in a row, where 16 heads' rows took
+// it 64 cycles of the address path.
+__device__ __forceinline__ int64_t qcat_at(const LatentParams& p, int b, int h, int c) {
+  if (!p.qsteps) return (static_cast<int64_t>(b) * p.H + h) * (p.R + p.rot) + c;
+  return ((static_cast<int64_t>(b) * ((p.H + 15) >> 4) + (h >> 4)) * p.qsteps + (c >> 5)) * 512 + (((c >> 3 & 3) << 4) + (h & 15)) * 8 + (c & 7);
+}
+
+// the rotated part of one head's queries, two rows' worth of loads in flight per lane
+template <typename T>
+__device__ __forceinline__ void absorb_rotated(const LatentParams& p, int h) {
+  const int dq = p.dim + p.rot, half = p.rot >> 1;
+  const T* Q = static_cast<const T*>(p.q) + h * dq + p.dim;
+  T* out = static_cast<T*>(p.qcat);
+  const int64_t newest = min(p.slot[0], static_cast<int64_t>(p.tcap - 1));
+  for (int i = threadIdx.x; i < p.B * half; i += 256) {  // both halves of a pair
+    const int b = i / half, d = i % half;
+    const int64_t pos = max(newest - (p.kv_start ? p.kv_start[b] : 0), static_cast<int64_t>(0));
+    const T* q = Q + static_cast<int64_t>(b) * p.H * dq;
+    const float u = to_f<T>(q[d]), v = to_f<T>(q[d + half]), c = p.cos_t[pos * half + d], s = p.sin_t[pos * half + d];
+    out[qcat_at(p, b, h, p.R + d)] = from_f<T>(u * c - v * s);
+    out[qcat_at(p, b, h, p.R + d + half)] = from_f<T>(v * c + u * s);
+  }
+}
+
 template <typename T, int VEC>
 __global__ __launch_bounds__(256) void latent_absorb_kernel(LatentParams p) {
   __shared__ float red[32][4][66];
   const int h = blockIdx.x, r0 = blockIdx.y * 64;
-  const int dq = p.dim + p.rot, lq = p.R + p.rot, half = p.rot >> 1;
+  if (r0 >= p.R) return absorb_rotated<T>(p, h);
+  const int dq = p.dim + p.rot;
   const int cg = threadIdx.x & 7, dg = threadIdx.x >> 3;
   const T* W = static_cast<const T*>(p.kv_up) + static_cast<int64_t>(h) * p.dim * p.R;
   const T* Q = static_cast<const T*>(p.q) + h * dq;
-  T* out = static_cast<T*>(p.qcat) + static_cast<int64_t>(h) * lq;
-  const int64_t qsb = static_cast<int64_t>(p.H) * dq, osb = static_cast<int64_t>(p.H) * lq;
+  T* out = static_cast<T*>(p.qcat);
+  const int64_t qsb = static_cast<int64_t>(p.H) * dq;
   for (int b0 = 0; b0 < p.B; b0 += 4) {
     float acc[4][8];
 #pragma unroll
@@ -268,36 +330,31 @@ __global__ __launch_bounds__(256) void latent_absorb_kernel(LatentParams p) {
     float s = 0.f;
 #pragma unroll
     for (int j = 0; j < 32; ++j) s += red[j][b][c];
-    if (b0 + b < p.B && r0 + c < p.R) out[(b0 + b) * osb + r0 + c] = from_f<T>(s);
+    if (b0 + b < p.B && r0 + c < p.R) out[qcat_at(p, b0 + b, h, r0 + c)] = from_f<T>(s);
     __syncthreads();
-  }
-  if (blockIdx.y == 0) {
-    for (int i = threadIdx.x; i < p.B * p.rot; i += 256) {
-      const int b = i / p.rot, d = i % p.rot;
-      const int64_t pos = max(min(p.slot[0], static_cast<int64_t>(p.tcap - 1)) - (p.kv_start ? p.kv_start[b] : 0), static_cast<int64_t>(0));
-      float v;
-      load_rotated<T, 1>(Q + b * qsb + p.dim, d, p.rot, p.cos_t + pos * half, p.sin_t + pos * half, &v);
-      out[b * osb + p.R + d] = from_f<T>(v);
-    }
   }
 }
 
 // The same on MFMA (bf16, dim <= 256, dim, rot and R multiples of 8): the head's [dim, 64] piece of W_uk
 // is staged as rows in LDS and read back transposed; wave w owns 16 of the 64 columns, batch rows
-// ride on the MFMA's row dimension.
+// ride on the MFMA's row dimension, 32 at a time, staged in LDS too (16 lanes on 16 rows would hold the address path
+// for 64 cycles a load, in each of the four waves).
 typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
 template <int ND>
 __global__ __launch_bounds__(256) void latent_absorb_mfma_kernel(LatentParams p) {
   constexpr int SW = 64 + 24;  // row stride: odd multiple of 16 B, 4 rows' 32-byte pieces on distinct banks
+  constexpr int SQ = 32 * ND + 8, NQ = ND / 2;  // query row stride; 16-byte pieces per thread of 32 rows
   __shared__ __attribute__((aligned(16))) bf16_t ws[32 * ND * SW];
+  __shared__ __attribute__((aligned(16))) bf16_t qs[32 * SQ];
   const int h = blockIdx.x, r0 = blockIdx.y * 64;
-  const int dq = p.dim + p.rot, lq = p.R + p.rot, half = p.rot >> 1;
+  if (r0 >= p.R) return absorb_rotated<bf16_t>(p, h);
+  const int dq = p.dim + p.rot;
   const bf16_t* W = static_cast<const bf16_t*>(p.kv_up) + static_cast<int64_t>(h) * p.dim * p.R;
   const bf16_t* Q = static_cast<const bf16_t*>(p.q) + h * dq;
-  bf16_t* out = static_cast<bf16_t*>(p.qcat) + static_cast<int64_t>(h) * lq;
-  const int64_t qsb = static_cast<int64_t>(p.H) * dq, osb = static_cast<int64_t>(p.H) * lq;
+  bf16_t* out = static_cast<bf16_t*>(p.qcat);
+  const int64_t qsb = static_cast<int64_t>(p.H) * dq;
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
-  bf16x8 reg[ND];
+  bf16x8 reg[ND], qreg[NQ];
 #pragma unroll
   for (int j = 0; j < ND; ++j) {
     const int i = threadIdx.x + 256 * j, d = i >> 3, c = r0 + (i & 7) * 8;
@@ -305,14 +362,13 @@ __global__ __launch_bounds__(256) void latent_absorb_mfma_kernel(LatentParams p)
     if (d < p.dim && c < p.R) v = load_bf16x8(W + static_cast<int64_t>(d) * p.R + c);
     reg[j] = v;
   }
-  s16x8 qf[ND];
   auto load_q = [&](int b0) {
 #pragma unroll
-    for (int k = 0; k < ND; ++k) {
-      const int d = 32 * k + 8 * g;
+    for (int j = 0; j < NQ; ++j) {
+      const int i = threadIdx.x + 256 * j, b = b0 + i / (4 * ND), d = i % (4 * ND) * 8;
       bf16x8 v = {0, 0, 0, 0, 0, 0, 0, 0};
-      if (d < p.dim) v = load_bf16x8(Q + min(b0 + r, p.B - 1) * qsb + d);
-      qf[k] = __builtin_bit_cast(s16x8, v);
+      if (b < p.B && d < p.dim) v = load_bf16x8(Q + b * qsb + d);
+      qreg[j] = v;
     }
   };
   load_q(0);
@@ -321,30 +377,33 @@ __global__ __launch_bounds__(256) void latent_absorb_mfma_kernel(LatentParams p)
     const int i = threadIdx.x + 256 * j;
     store_bf16x8(ws + (i >> 3) * SW + (i & 7) * 8, reg[j]);
   }
-  __syncthreads();
-  for (int b0 = 0; b0 < p.B; b0 += 16) {
-    if (b0) load_q(b0);
-    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+  for (int b0 = 0; b0 < p.B; b0 += 32) {
+    if (b0) __syncthreads();  // every wave has read the last rows
+#pragma unroll
+    for (int j = 0; j < NQ; ++j) {
+      const int i = threadIdx.x + 256 * j;
+      store_bf16x8(qs + i / (4 * ND) * SQ + i % (4 * ND) * 8, qreg[j]);
+    }
+    __syncthreads();
+    if (b0 + 32 < p.B) load_q(b0 + 32);
+    f32x4 acc[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
 #pragma unroll
     for (int k = 0; k < ND; ++k) {
       const bf16_t* wp = ws + (32 * k + 8 * g + ((lane & 15) >> 2)) * SW + 16 * wave + 4 * (lane & 3);
       const s16x4 a = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(wp));
       const s16x4 c = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(wp + 4 * SW));
-      acc = Mma<bf16_t>::mma(qf[k], s16x8{a[0], a[1], a[2], a[3], c[0], c[1], c[2], c[3]}, acc);
+      const s16x8 w = {a[0], a[1], a[2], a[3], c[0], c[1], c[2], c[3]};
+#pragma unroll
+      for (int t = 0; t < 2; ++t) acc[t] = Mma<bf16_t>::mma(Mma<bf16_t>::row(qs + (16 * t + r) * SQ + 32 * k + 8 * g), w, acc[t]);
     }
     const int col = r0 + 16 * wave + r;
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-      if (b0 + 4 * g + i < p.B && col < p.R) out[(b0 + 4 * g + i) * osb + col] = f2bf(acc[i]);
-  }
-  if (blockIdx.y == 0) {
-    for (int i = threadIdx.x; i < p.B * p.rot; i += 256) {
-      const int b = i / p.rot, d = i % p.rot;
-      const int64_t pos = max(min(p.slot[0], static_cast<int64_t>(p.tcap - 1)) - (p.kv_start ? p.kv_start[b] : 0), static_cast<int64_t>(0));
-      float v;
-      load_rotated<bf16_t, 1>(Q + b * qsb + p.dim, d, p.rot, p.cos_t + pos * half, p.sin_t + pos * half, &v);
-      out[b * osb + p.R + d] = f2bf(v);
-    }
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int b = b0 + 16 * t + 4 * g + i;
+        if (b < p.B && col < p.R) out[qcat_at(p, b, h, col)] = f2bf(acc[t][i]);
+      }
   }
 }
 
@@ -486,63 +545,98 @@ int64_t decode_lds(const LatentParams& p, int BN) {
 }
 
 // ------------------------------------------------------------------------------------ combine
-// grid (H, B, ceil(vdim / kCombV)), 256 threads: o[b][h] = W_uv[h] (sum over splits). ns <= 256.
+// grid (H, ceil(B / BB), ceil(vdim / kCombV)), 256 threads: o[b][h] = W_uv[h] (sum over splits), BB rows of the batch per
+// workgroup. ns <= 256. Everything that does not depend on the splits' weights is loaded before they are formed
+// (one wave per row does that): this wave's W_uv rows, the partial outputs' first splits.
 constexpr int kCombV = 32;
-template <typename T, int VEC>
+template <typename T, int VEC, int BB>
 __global__ __launch_bounds__(256) void latent_combine_kernel(LatentParams p) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-  float* os = reinterpret_cast<float*>(smem);  // [R]
-  __shared__ float ws[256];
-  __shared__ float scratch[4];
-  const int h = blockIdx.x, b = blockIdx.y, tid = threadIdx.x;
-  const int64_t pb = (static_cast<int64_t>(b) * p.H + h) * p.ns;
-  // independent of everything below: the first piece of this wave's W_uv rows, the first splits
-  const T* W = static_cast<const T*>(p.kv_up) + (static_cast<int64_t>(p.H) * p.dim + static_cast<int64_t>(h) * p.vdim) * p.R;
+  float* os = reinterpret_cast<float*>(smem);  // [BB][R]
+  __shared__ float ws[BB][256];
+  const int h = blockIdx.x, b0 = blockIdx.y * BB, tid = threadIdx.x;
   const int wave = tid >> 6, lane = tid & 63;
-  constexpr int U = kCombV / 4;
+  constexpr int U = kCombV / 4, PRE = 16 / BB;
+  const T* W = static_cast<const T*>(p.kv_up) + (static_cast<int64_t>(p.H) * p.dim + static_cast<int64_t>(h) * p.vdim) * p.R;
   const int v0 = blockIdx.z * kCombV + wave * U;
+  auto pair = [&](int j) { return (static_cast<int64_t>(min(b0 + j, p.B - 1)) * p.H + h) * p.ns; };
+  float m[4], l[4];
+  if (wave < BB) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int s = lane + 64 * u;
+      m[u] = s < p.ns ? p.part_ml[(pair(wave) + s) * 2] : -INFINITY;
+      l[u] = s < p.ns ? p.part_ml[(pair(wave) + s) * 2 + 1] : 0.f;
+    }
+  }
+  float x[BB][PRE][2];
+#pragma unroll
+  for (int j = 0; j < BB; ++j)
+#pragma unroll
+    for (int s = 0; s < PRE; ++s)
+#pragma unroll
+      for (int e = 0; e < 2; ++e)
+        x[j][s][e] = s < p.ns && tid + 256 * e < p.R ? p.part_o[(pair(j) + s) * p.R + tid + 256 * e] : 0.f;  // (empty splits hold zeros)
   float wv[U][VEC];
   auto load_w = [&](int c) {
 #pragma unroll
     for (int u = 0; u < U; ++u) load_vec<T, VEC>(W + static_cast<int64_t>(min(v0 + u, p.vdim - 1)) * p.R + c, wv[u]);
   };
   if (lane * VEC < p.R) load_w(lane * VEC);
-  const float m = tid < p.ns ? p.part_ml[(pb + tid) * 2] : -INFINITY;
-  const float l0 = tid < p.ns ? p.part_ml[(pb + tid) * 2 + 1] : 0.f;
-  const float mx = block_max<256>(m, scratch);
-  const float w = m == -INFINITY ? 0.f : exp2f(m - mx);
-  const float l = block_sum<256>(w * l0, scratch);
-  ws[tid] = l > 0.f ? w / l : 0.f;
-  __syncthreads();
-  for (int c = tid; c < p.R; c += 256) {
-    float v = 0.f;
-    int s = 0;
-    for (; s + 16 <= p.ns; s += 16) {  // (empty splits hold zeros)
-      float x[16];
+  if (wave < BB) {
+    const float mx = wave_max(fmaxf(fmaxf(m[0], m[1]), fmaxf(m[2], m[3])));
+    float w[4], sum = 0.f;
 #pragma unroll
-      for (int u = 0; u < 16; ++u) x[u] = p.part_o[(pb + s + u) * p.R + c];
-#pragma unroll
-      for (int u = 0; u < 16; ++u) v += ws[s + u] * x[u];
+    for (int u = 0; u < 4; ++u) {
+      w[u] = m[u] == -INFINITY ? 0.f : exp2f(m[u] - mx);
+      sum += w[u] * l[u];
     }
-    for (; s < p.ns; ++s) v += ws[s] * p.part_o[(pb + s) * p.R + c];
-    os[c] = v;
+    sum = wave_sum(sum);
+#pragma unroll
+    for (int u = 0; u < 4; ++u) ws[wave][lane + 64 * u] = sum > 0.f ? w[u] / sum : 0.f;
   }
   __syncthreads();
-  T* O = static_cast<T*>(p.o) + (static_cast<int64_t>(b) * p.H + h) * p.vdim;
-  float acc[U];
 #pragma unroll
-  for (int u = 0; u < U; ++u) acc[u] = 0.f;
+  for (int j = 0; j < BB; ++j) {
+    float v[2] = {0.f, 0.f};
+#pragma unroll
+    for (int u = 0; u < PRE; ++u)
+#pragma unroll
+      for (int e = 0; e < 2; ++e) v[e] += ws[j][u] * x[j][u][e];
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      const int c = tid + 256 * e;
+      for (int s = PRE; s < p.ns && c < p.R; ++s) v[e] += ws[j][s] * p.part_o[(pair(j) + s) * p.R + c];
+      if (c < p.R) os[j * p.R + c] = v[e];
+    }
+  }
+  for (int c = tid + 512; c < p.R; c += 256)
+    for (int j = 0; j < BB; ++j) {
+      float v = 0.f;
+      for (int s = 0; s < p.ns; ++s) v += ws[j][s] * p.part_o[(pair(j) + s) * p.R + c];
+      os[j * p.R + c] = v;
+    }
+  __syncthreads();
+  float acc[BB][U];
+#pragma unroll
+  for (int j = 0; j < BB; ++j)
+#pragma unroll
+    for (int u = 0; u < U; ++u) acc[j][u] = 0.f;
   for (int c = lane * VEC; c < p.R; c += 64 * VEC) {
     if (c != lane * VEC) load_w(c);
 #pragma unroll
-    for (int u = 0; u < U; ++u)
+    for (int j = 0; j < BB; ++j)
 #pragma unroll
-      for (int e = 0; e < VEC; ++e) acc[u] += wv[u][e] * os[c + e];
+      for (int u = 0; u < U; ++u)
+#pragma unroll
+        for (int e = 0; e < VEC; ++e) acc[j][u] += wv[u][e] * os[j * p.R + c + e];
   }
 #pragma unroll
-  for (int u = 0; u < U; ++u) {
-    const float s = wave_sum(acc[u]);
-    if (lane == 0 && v0 + u < p.vdim) O[v0 + u] = from_f<T>(s);
+  for (int j = 0; j < BB; ++j) {
+    const float s = step_reduce<64>(acc[j]);
+    const int v = v0 + (lane >> 3);
+    if ((lane & 7) == 0 && v < p.vdim && b0 + j < p.B)
+      static_cast<T*>(p.o)[(static_cast<int64_t>(b0 + j) * p.H + h) * p.vdim + v] = from_f<T>(s);
   }
 }
 
@@ -582,20 +676,28 @@ void attend_any(const LatentParams& p, int BN, hipStream_t st) {
 }
 
 template <typename T>
-void decode(const LatentParams& p, int BN, hipStream_t st) {
+void decode(const LatentParams& in, int BN, hipStream_t st) {
+  LatentParams p = in;
+  const bool mfma = sizeof(T) == 2 && latent_decode_mfma_ok(p);
+  p.qsteps = mfma ? latent_decode_mfma_steps(p) : 0;
   const bool vec = p.R % 8 == 0 && reinterpret_cast<uintptr_t>(p.kv_up) % 16 == 0;
-  const dim3 ga(p.H, (p.R + 63) / 64);
+  const dim3 ga(p.H, (p.R + 63) / 64 + 1);
   if (sizeof(T) == 2 && vec && p.dim % 8 == 0 && p.rot % 8 == 0 && p.dim <= 256 && reinterpret_cast<uintptr_t>(p.q) % 16 == 0) {
     if (p.dim <= 64) latent_absorb_mfma_kernel<2><<<ga, 256, 0, st>>>(p);
     else if (p.dim <= 128) latent_absorb_mfma_kernel<4><<<ga, 256, 0, st>>>(p);
     else latent_absorb_mfma_kernel<8><<<ga, 256, 0, st>>>(p);
   } else if (vec) latent_absorb_kernel<T, 8><<<ga, 256, 0, st>>>(p);
   else latent_absorb_kernel<T, 1><<<ga, 256, 0, st>>>(p);
-  if (sizeof(T) == 2 && latent_decode_mfma_ok(p)) launch_latent_decode_mfma(p, st);
+  if (mfma) launch_latent_decode_mfma(p, st);
   else attend_any<T>(p, BN, st);
-  const dim3 gc(p.H, p.B, (p.vdim + kCombV - 1) / kCombV);
-  if (vec) latent_combine_kernel<T, 8><<<gc, 256, 4 * p.R, st>>>(p);
-  else latent_combine_kernel<T, 1><<<gc, 256, 4 * p.R, st>>>(p);
+  // Four rows share a read of W_uv once 512 workgroups are left (B = 32, 16 heads of 128: 8.0 us against 15.7 a row at a time)
+  const int nv = (p.vdim + kCombV - 1) / kCombV;
+  const bool four = p.H * ((p.B + 3) / 4) * nv >= 512 && 16ll * p.R <= 32 * 1024;
+  const dim3 gc(p.H, four ? (p.B + 3) / 4 : p.B, nv);
+  if (four && vec) latent_combine_kernel<T, 8, 4><<<gc, 256, 16 * p.R, st>>>(p);
+  else if (four) latent_combine_kernel<T, 1, 4><<<gc, 256, 16 * p.R, st>>>(p);
+  else if (vec) latent_combine_kernel<T, 8, 1><<<gc, 256, 4 * p.R, st>>>(p);
+  else latent_combine_kernel<T, 1, 1><<<gc, 256, 4 * p.R, st>>>(p);
 }
 
 }  // namespace

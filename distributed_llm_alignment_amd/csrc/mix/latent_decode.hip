@@ -57,12 +57,12 @@ __global__ __launch_bounds__(256, 2) void latent_decode_mfma_kernel(LatentParams
   if (k0 < k1) load_tile(k0);
   s16x8 qf[NK];
   {
-    const bf16_t* Q = static_cast<const bf16_t*>(p.qcat) + (static_cast<int64_t>(b) * p.H + h0 + min(r, nh - 1)) * lq;
+    // (rows of a group beyond its heads hold anything: it stays in their own outputs, which are not stored)
+    const bf16_t* Q = static_cast<const bf16_t*>(p.qcat) + (static_cast<int64_t>(b) * gridDim.y + blockIdx.y) * (NK * 512) + lane * 8;
 #pragma unroll
     for (int k = 0; k < NK; ++k) {
-      const int d = 32 * k + 8 * g;
       bf16x8 v = {0, 0, 0, 0, 0, 0, 0, 0};
-      if (d < lq) v = load_bf16x8(Q + d);
+      if (32 * k + 8 * g < lq) v = load_bf16x8(Q + k * 512);
       qf[k] = __builtin_bit_cast(s16x8, v);
     }
   }
@@ -164,10 +164,14 @@ bool latent_decode_mfma_ok(const LatentParams& p) {
          reinterpret_cast<uintptr_t>(p.latent) % 16 == 0 && reinterpret_cast<uintptr_t>(p.qcat) % 16 == 0;
 }
 
-void launch_latent_decode_mfma(const LatentParams& p, hipStream_t st) {
+int latent_decode_mfma_steps(const LatentParams& p) {
   const int w = p.R + p.rot;
-  if (w <= 192 && p.R <= 128) go<6, 2>(p, st);
-  else if (w <= 320 && p.R <= 256) go<10, 4>(p, st);
+  return w <= 192 && p.R <= 128 ? 6 : w <= 320 && p.R <= 256 ? 10 : 18;
+}
+
+void launch_latent_decode_mfma(const LatentParams& p, hipStream_t st) {
+  if (p.qsteps == 6) go<6, 2>(p, st);
+  else if (p.qsteps == 10) go<10, 4>(p, st);
   else go<18, 8>(p, st);
 }
 

@@ -34,7 +34,8 @@ struct LatentParams {
   const void* latent;     // decode: cache [B, Tmax, R + rot]
   int64_t l_sb, l_st;
   const void* kv_up;      // decode: [H (dim + vdim), R]
-  void* qcat;             // decode: [B, H, R + rot] query in latent space | rotated part
+  void* qcat;             // decode: [B, H, R + rot] query in latent space | rotated part (order: qcat_at)
+  int qsteps;             // decode: 32-wide steps of the MFMA kernel's order of qcat, 0: rows
   void* o;                // [B, T, H vdim]
   float* part_o;          // decode: [B, H, ns, R]
   float* part_ml;         // decode: [B, H, ns, 2]

@@ -28,21 +28,15 @@ __device__ __forceinline__ void step_load(const float* S, int r0, int vhi, int d
 
 // acc[u] summed over a group's LPR >= 8 lanes; a lane returns row (lane's top three bits)'s sum
 template <int LPR>
-__device__ __forceinline__ float step_reduce(float (&acc)[kStepRows]) {
+__device__ __forceinline__ float step_reduce(const float (&acc)[kStepRows]) {
   const int li = threadIdx.x % LPR;
-  int n = kStepRows;
+  const bool u4 = li & LPR / 2, u2 = li & LPR / 4, u1 = li & LPR / 8;
+  float a[4], b[2];
 #pragma unroll
-  for (int o = LPR / 2; o >= LPR / 8; o >>= 1) {
-    n >>= 1;
-    const bool up = li & o;
+  for (int j = 0; j < 4; ++j) a[j] = (u4 ? acc[j + 4] : acc[j]) + __shfl_xor(u4 ? acc[j] : acc[j + 4], LPR / 2, 64);
 #pragma unroll
-    for (int j = 0; j < kStepRows / 2; ++j) {
-      if (j >= n) continue;
-      const float mine = up ? acc[j + n] : acc[j], other = up ? acc[j] : acc[j + n];
-      acc[j] = mine + __shfl_xor(other, o, 64);
-    }
-  }
-  float v = acc[0];
+  for (int j = 0; j < 2; ++j) b[j] = (u2 ? a[j + 2] : a[j]) + __shfl_xor(u2 ? a[j] : a[j + 2], LPR / 4, 64);
+  float v = (u1 ? b[1] : b[0]) + __shfl_xor(u1 ? b[0] : b[1], LPR / 8, 64);
 #pragma unroll
   for (int o = LPR / 16; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
   return v;

@@ -1,5 +1,5 @@
-"""One decoded token of retention and gated linear attention: sizes at the edges of the kernels' lanes and rows, states
-split over workgroups, both element types, against the CPU forms."""
+"""One decoded token of retention, gated linear attention and latent attention: sizes at the edges of the kernels' lanes,
+rows and tiles, states split over workgroups, both element types, against the CPU forms."""
 import pytest
 import torch
 
@@ -56,3 +56,26 @@ def test_gla_step(B, H, dim, vdim, rank, dtype):
         out[dev] = ops.gla.decode(*t, H, dim, vdim, 8.0, EPS, s, slot.to(dev), None, base=33), s
     close(out["cuda"][0], out["cpu"][0], dtype)
     close(out["cuda"][1], out["cpu"][1], torch.float32)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("B,H,dim,rot,vdim,R", [
+    (33, 16, 128, 64, 128, 512),  # four rows a workgroup in the merge, a last group of one, two passes of query rows
+    (5, 3, 64, 16, 40, 128), (2, 17, 256, 32, 32, 256),  # groups of heads that are not full, the smaller and largest tiles
+    (3, 2, 24, 0, 20, 72), (2, 2, 20, 6, 33, 1000)])  # no rotated part; odd sizes, more than 512 columns
+def test_latent_step(B, H, dim, rot, vdim, R, dtype):
+    """bf16: queries in latent space and the result are rounded, scores and weights are not (one more 2^-8)."""
+    g = torch.Generator().manual_seed(B + R)
+    q = torch.randn(B, 1, H * (dim + rot), generator=g).to(dtype)
+    latent = torch.randn(B, 150, R + rot, generator=g).to(dtype)
+    up = (torch.randn(H * (dim + vdim), R, generator=g) * R ** -0.5).to(dtype)
+    ang = torch.rand(150, rot // 2, generator=g) * 6.3
+    start, slot = torch.randint(0, 60, (B,), generator=g).int(), torch.tensor([130])
+    out = {}
+    for dev in ("cpu", "cuda"):
+        t = [x.to(dev).float() if dev == "cpu" else x.to(dev) for x in (q, latent, up)]
+        out[dev] = ops.latent.decode(*t, H, dim, rot, vdim, (dim + rot) ** -0.5, 100, slot.to(dev), start.to(dev),
+                                     ang.cos().to(dev), ang.sin().to(dev), base=130)
+    want = out["cpu"].double()
+    off = float((out["cuda"].cpu().double() - want).norm())
+    assert off <= (8e-3 if dtype == torch.bfloat16 else 2e-5) * float(want.norm())
