@@ -208,19 +208,37 @@ __global__ __launch_bounds__(64) void chunk_decode_any_kernel(ChunkAttnParams p)
 // grid (H, B), 256 threads: o = sum_s 2^(m_s - m) o_s / sum_s 2^(m_s - m) l_s (ns <= 256)
 template <typename T>
 __global__ __launch_bounds__(256) void chunk_combine_kernel(ChunkAttnParams p) {
-  __shared__ float scratch[4], ws[256];
+  __shared__ float ws[256];
   const int64_t bh = static_cast<int64_t>(blockIdx.y) * p.H + blockIdx.x;
-  const bool in = static_cast<int>(threadIdx.x) < p.ns;
-  const float m = in ? p.part_ml[2 * (bh * p.ns + threadIdx.x)] : -INFINITY;
-  const float l = in ? p.part_ml[2 * (bh * p.ns + threadIdx.x) + 1] : 0.f;
-  const float mx = block_max<256>(m, scratch);
-  const float w = m == -INFINITY ? 0.f : exp2f(m - mx);
-  const float total = block_sum<256>(w * l, scratch);
-  ws[threadIdx.x] = w;
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  constexpr int PRE = 8;  // the first splits' outputs leave before the weights are formed
+  float x[PRE], m[4], l[4];
+#pragma unroll
+  for (int s = 0; s < PRE; ++s) x[s] = s < p.ns && tid < p.vdim ? p.part_o[(bh * p.ns + s) * p.vdim + tid] : 0.f;
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {  // (every wave forms the sum, the first one stores the weights)
+    const int s = lane + 64 * u;
+    m[u] = s < p.ns ? p.part_ml[2 * (bh * p.ns + s)] : -INFINITY;
+    l[u] = s < p.ns ? p.part_ml[2 * (bh * p.ns + s) + 1] : 0.f;
+  }
+  const float mx = wave_max(fmaxf(fmaxf(m[0], m[1]), fmaxf(m[2], m[3])));
+  float total = 0.f;
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    const float w = m[u] == -INFINITY ? 0.f : exp2f(m[u] - mx);
+    total += w * l[u];
+    if (wave == 0) ws[lane + 64 * u] = w;
+  }
+  total = wave_sum(total);
   __syncthreads();
-  for (int v = threadIdx.x; v < p.vdim; v += 256) {
+  for (int v = tid; v < p.vdim; v += 256) {
     float o = 0.f;
-    for (int s = 0; s < p.ns; ++s)
+    int s = 0;
+    if (v == tid) {
+#pragma unroll
+      for (; s < PRE; ++s) o += ws[s] != 0.f ? ws[s] * x[s] : 0.f;
+    }
+    for (; s < p.ns; ++s)
       if (ws[s] != 0.f) o += ws[s] * p.part_o[(bh * p.ns + s) * p.vdim + v];
     static_cast<T*>(p.o)[bh * p.vdim + v] = from_f<T>(o / total);
   }

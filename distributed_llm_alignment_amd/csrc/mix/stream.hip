@@ -55,13 +55,14 @@ __global__ __launch_bounds__(NT) void stream_norm_kernel(float* __restrict__ x, 
     for (int e = 0; e < 4; ++e) dv[j][e] = 0.f;
     if (c < H && delta) load_vec<T, 4>(delta + base + c, dv[j]);
   }
-  float wv[NV][4], iv[NV][4];
+  float wv[NV][4], iv[NV][4], dw[NV][4];
 #pragma unroll
   for (int j = 0; j < NV; ++j) {  // (in flight behind the sums)
     const int c = 4 * (threadIdx.x + NT * j);
     if (c < H && w) load_vec<T, 4>(w + c, wv[j]);
 #pragma unroll
-    for (int e = 0; e < 4; ++e) iv[j][e] = 0.f;
+    for (int e = 0; e < 4; ++e) iv[j][e] = dw[j][e] = 0.f;
+    if (c < H && delta_w) load_vec<T, 4>(delta_w + c, dw[j]);
     if (c < H && inject) load_vec<float, 4>(inject + base + c, iv[j]);
   }
   if (delta_w) {
@@ -72,15 +73,9 @@ __global__ __launch_bounds__(NT) void stream_norm_kernel(float* __restrict__ x, 
       for (int e = 0; e < 4; ++e) ss += dv[j][e] * dv[j][e];
     const float r = rsqrtf(row_sum<NT>(ss, scratch) / H + eps);
 #pragma unroll
-    for (int j = 0; j < NV; ++j) {
-      const int c = 4 * (threadIdx.x + NT * j);
-      if (c < H) {
-        float dw[4];
-        load_vec<T, 4>(delta_w + c, dw);
+    for (int j = 0; j < NV; ++j)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) dv[j][e] *= r * dw[e];
-      }
-    }
+      for (int e = 0; e < 4; ++e) dv[j][e] *= r * dw[j][e];
   }
   float ss = 0.f;
 #pragma unroll

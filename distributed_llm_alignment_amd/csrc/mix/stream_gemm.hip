@@ -106,6 +106,7 @@ __global__ __launch_bounds__(64 * WV) void stream_gemm_kernel(StreamGemmParams p
   };
   float xv[NO], cv[NO];  // the stream's value; the gate's factor or the bias
   bf16_t nw[NO], rw[NO];
+  int64_t id[EPI == kGate ? NO : 1];
 #pragma unroll
   for (int o = 0; o < NO; ++o) {
     int ti, m, n;
@@ -120,10 +121,7 @@ __global__ __launch_bounds__(64 * WV) void stream_gemm_kernel(StreamGemmParams p
       if (ok && p.res_ssq) rw[o] = p.res_w[n];
       if (ok && p.bias) cv[o] = bf2f(p.bias[n]);
     }
-    if constexpr (EPI == kGate) {
-      const int64_t id = ok ? p.ids[m] : -1;
-      if (id >= 0 && id < p.vocab) cv[o] = bf2f(p.table[id * p.ldt + p.off + n]);
-    }
+    if constexpr (EPI == kGate) id[o] = ok ? p.ids[m] : -1;
   }
   RowScales<MT, WV> in_scale, res_scale;
   if (p.ssq_in) in_scale.load(p.ssq_in, p.nssq, p.M);
@@ -132,6 +130,14 @@ __global__ __launch_bounds__(64 * WV) void stream_gemm_kernel(StreamGemmParams p
   }
 #pragma unroll
   for (int d = 0; d < D; ++d) issue(s0 + d, d);  // (a wave with fewer stages brings what it does not read)
+  if constexpr (EPI == kGate) {  // (needs the ids: behind the first stages, not in front of them)
+#pragma unroll
+    for (int o = 0; o < NO; ++o) {
+      int ti, m, n;
+      place(o, ti, m, n);
+      if (id[o] >= 0 && id[o] < p.vocab) cv[o] = bf2f(p.table[id[o] * p.ldt + p.off + n]);
+    }
+  }
   if (p.ssq_in) in_scale.to(rstd, p.ssq_in, p.nssq, p.M, p.K, p.eps);
   if constexpr (EPI == kPost) {
     if (p.res_ssq) res_scale.to(rres, p.res_ssq, p.nres, p.M, p.N, p.eps);
@@ -250,9 +256,10 @@ enum Tile { kT8, kT16, kT16Deep, kT32, kT64 };
 //   below K = 2048 there is nothing to share out: 2048 x 128 2.6 / 2.5 / 2.7 / 3.4 against 2.4 / 2.3 / 2.3 / 3.4);
 //   32 columns from 17 rows on for more tiles than CUs (8192 x 2048: 10.1 / 11.9 at 32 / 48 rows against 14.4 / 17.6
 //   with 16), and at 9 to 16 rows from 320 tiles on (5120 x 2048: 6.9 against 7.9);
-//   64 columns from 33 rows on for 1024 tiles (16384 x 4096: 26.4 against 35.3 at 48 rows).
+//   64 columns from 33 rows on where 32 would not fit the CUs at once (16384 x 4096: 26.4 against 35.3 at 48 rows).
 // Four waves with deeper rings instead of eight take long rows (4096 x 16384: 27.6 / 28.8 / 35.2 / 43.3 against 31.3 /
-// 31.7 / 44.4 / 48.2) and, with few rows, many tiles (32000 x 2048: 21.7 against 23.7).
+// 31.7 / 44.4 / 48.2) and, with few rows, many tiles (32000 x 2048: 21.7 against 23.7); two workgroups of them fit a
+// CU where one of eight does, which decides at 17 to 32 rows beyond 256 workgroups (8208 x 2048: 257 of them).
 Tile choose(const StreamGemmParams& p, int epi) {
   const int tiles = (p.N + 15) / 16, M = p.M;
   if (epi == kGeglu) return M <= 16 ? kT16Deep : kT32;
@@ -260,7 +267,7 @@ Tile choose(const StreamGemmParams& p, int epi) {
   if (p.K >= 8192) return kT16Deep;
   if (M <= 8) return tiles >= 1024 && p.K <= 2048 ? kT16Deep : kT16;
   if (M <= 16) return tiles >= 320 ? kT32 : kT16;
-  if (M > 32 && tiles >= 1024) return kT64;
+  if (M > 32 && tiles > 512) return kT64;
   return tiles > 256 ? kT32 : kT16;
 }
 
@@ -295,7 +302,7 @@ void launch(const StreamGemmParams& p, Tile t, hipStream_t st) {
         else go<8, 16, 1, 2, 4, EPI>(p, st);
       } else if (t == kT32) {
         if (M <= 16) go<2, 16, 2, 3, 4, EPI>(p, st);
-        else if (M <= 32 && p.N >= 16 * 1024) go<4, 16, 2, 2, 4, EPI>(p, st);
+        else if (M <= 32 && p.N > 32 * 256) go<4, 16, 2, 2, 4, EPI>(p, st);
         else if (M <= 32) go<4, 16, 2, 2, 8, EPI>(p, st);
         else if (M <= 48) go<6, 16, 2, 1, 8, EPI>(p, st);
         else go<8, 16, 2, 1, 8, EPI>(p, st);
