@@ -43,6 +43,18 @@ def _ref_linear_logprob(hidden, weight, targets):
     return torch.where(targets >= 0, lp, torch.zeros_like(lp))
 
 
+def _logits(hidden: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
+    """hidden @ weight^T with rows that start at multiples of 128 bytes, whatever the vocabulary is: with GPT-2's 50257
+    columns side by side every row starts elsewhere, and the products around the logits (8000 rows, width 768)
+    take 662 / 833 / 768 us (logits, their two gradients) against 544 / 800 / 631 with rows of 50304. Small heads
+    gain nothing on the GPU and pay the calls below on the host."""
+    V = weight.shape[0]
+    if V % 64 == 0 or V < 8192 or hidden.dtype != torch.bfloat16 or weight.dtype != torch.bfloat16:
+        return F.linear(hidden, weight)
+    out = torch.empty((hidden.shape[0], V + -V % 64), dtype=hidden.dtype, device=hidden.device)[:, :V]
+    return torch.mm(hidden, weight.t(), out=out)
+
+
 class _LinearLogprobFn(torch.autograd.Function):
     @staticmethod
     def forward(ctx, hidden, weight, targets):
@@ -50,7 +62,7 @@ class _LinearLogprobFn(torch.autograd.Function):
         need_grad = ctx.needs_input_grad[0] or ctx.needs_input_grad[1]
         N = hidden.shape[0]
         if need_grad:
-            logits = F.linear(hidden, weight)
+            logits = _logits(hidden, weight)
             logp, lse = ops.logprob_fwd(logits, targets)
             ctx.save_for_backward(hidden, targets, lse, logits)
             ctx.weight = weight  # (on ctx: see ops.linear._LinearMainGradFn)
@@ -58,7 +70,7 @@ class _LinearLogprobFn(torch.autograd.Function):
         logp = torch.empty(N, dtype=torch.float32, device=hidden.device)
         for s in range(0, N, _NO_GRAD_CHUNK):
             e = min(N, s + _NO_GRAD_CHUNK)
-            lg = F.linear(hidden[s:e], weight)
+            lg = _logits(hidden[s:e], weight)
             lp, _ = ops.logprob_fwd(lg, targets[s:e])
             logp[s:e] = lp
         return logp

@@ -2,6 +2,8 @@
 import pytest
 import torch
 
+from distributed_llm_alignment_amd import ops
+
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
 
@@ -30,3 +32,46 @@ def test_adamw_sizes(n, grad_dtype):
     for k in want:
         torch.testing.assert_close(state[k].double(), want[k], rtol=2e-6, atol=2e-6)
     assert torch.equal(p[:n], state["w"][:n].bfloat16()) and not p[n:].any()
+
+
+@pytest.mark.parametrize("V,ld", [(8, 8), (1, 8), (777, 784), (2051, 2112), (2048, 2048), (50257, 50304), (777, 777), (1000, 1001)])
+def test_logprob_row_ends(V, ld):
+    """Rows with a padded stride, a vocabulary that is not a multiple of a piece, and unaligned rows: log-probabilities and
+    in-place gradients against float64 (fp32 sums; the bf16 gradient rounds by 2^-8), the padding left alone."""
+    from distributed_llm_alignment_amd.ops import _ext
+
+    g0 = torch.Generator(device=DEV).manual_seed(V)
+    N = 33
+    buf = (torch.randn(N, ld, generator=g0, device=DEV) * 3).bfloat16()
+    x, pad = buf[:, :V], buf[:, V:].clone()
+    z = x.double()
+    tgt = torch.randint(0, V, (N,), generator=g0, device=DEV)
+    tgt[3], tgt[4], tgt[5] = -100, V - 1, 0
+    gr = torch.randn(N, generator=g0, device=DEV)
+    lp, lse = _ext.require().logprob_fwd(x, tgt)
+    want = torch.where(tgt >= 0, torch.log_softmax(z, -1).gather(1, tgt.clamp(min=0)[:, None])[:, 0], 0)
+    torch.testing.assert_close(lse.double(), torch.logsumexp(z, -1), rtol=1e-5, atol=1e-5)
+    torch.testing.assert_close(lp.double(), want, rtol=1e-5, atol=2e-5)
+    _ext.require().logprob_bwd(x, tgt, lse, gr)
+    hot = torch.nn.functional.one_hot(tgt.clamp(min=0), V).double()
+    dz = (gr * (tgt >= 0)).double()[:, None] * (hot - z.softmax(-1))
+    assert float((x.double() - dz).norm()) <= 4e-3 * float(dz.norm()) + 1e-12
+    assert torch.equal(buf[:, V:], pad)
+
+
+@pytest.mark.parametrize("V", [97, 8191, 8193, 8256])
+def test_linear_logprob_padded_rows(V):
+    """The LM head over vocabularies that need padded rows and ones that do not, gradients included (float64; bf16 products)."""
+    g0 = torch.Generator(device=DEV).manual_seed(V)
+    h = torch.randn(40, 64, generator=g0, device=DEV).bfloat16().requires_grad_()
+    w = (torch.randn(V, 64, generator=g0, device=DEV) * 0.2).bfloat16().requires_grad_()
+    tgt, gr = torch.randint(0, V, (40,), generator=g0, device=DEV), torch.randn(40, generator=g0, device=DEV)
+    (ops.linear_logprob(h, w, tgt) * gr).sum().backward()
+    hd, wd = h.detach().double().requires_grad_(), w.detach().double().requires_grad_()
+    lp = torch.log_softmax(hd @ wd.T, -1).gather(1, tgt[:, None])[:, 0]
+    (lp * gr).sum().backward()
+    with torch.no_grad():
+        got = ops.linear_logprob(h, w, tgt)
+    assert float((got.double() - lp).norm()) <= 8e-3 * float(lp.norm())
+    for a, b in ((h, hd), (w, wd)):
+        assert float((a.grad.double() - b.grad).norm()) <= 2e-2 * float(b.grad.norm())
