@@ -32,6 +32,9 @@ int sample_split_chunks(const void*, int64_t, int64_t, int, float, int, float, b
 size_t sample_workspace_bytes(int64_t, int);
 void launch_sample_split(const void*, bool, int64_t, int64_t, int, int, float, int, float,
                          const int64_t*, int64_t*, void*, hipStream_t);
+void launch_token_step(const int64_t*, bool*, int64_t*, int64_t*, int64_t*, int64_t, int64_t, int64_t*, int64_t*, int64_t,
+                       int64_t, int, hipStream_t);
+void launch_kv_advance(int64_t*, int*, int*, int, hipStream_t);
 
 int skinny_splits(int M, int N, int K);
 bool skinny_use_ksplit(int N, int K);
@@ -724,6 +727,41 @@ at::Tensor sample_tokens(const at::Tensor& logits, double temperature, int64_t t
   return out;
 }
 
+static void check_flat(const at::Tensor& t, at::ScalarType type, int64_t n, const at::Tensor& like, const char* name) {
+  check_cuda(t, name);
+  TORCH_CHECK(t.scalar_type() == type && t.is_contiguous() && t.numel() == n && t.device() == like.device(), name, ": ",
+              n, " contiguous elements of ", type, " on the same device expected");
+}
+
+// bookkeeping after a draw (token_step_kernel): every buffer but `next` is updated in place
+void token_step(const at::Tensor& next, at::Tensor finished, at::Tensor tok, at::Tensor seq, at::Tensor mask,
+                at::Tensor col, at::Tensor rng, int64_t eos, int64_t pad) {
+  TORCH_CHECK(next.dim() == 1 && seq.dim() == 2 && mask.sizes() == seq.sizes(), "next [B], seq and mask [B, columns]");
+  const int64_t B = next.size(0);
+  TORCH_CHECK(B < (1ll << 31) && seq.size(0) == B, "token_step: rows");
+  check_flat(next, at::kLong, B, next, "next");
+  check_flat(finished, at::kBool, B, next, "finished");
+  check_flat(tok, at::kLong, B, next, "tok");
+  check_flat(seq, at::kLong, seq.numel(), next, "seq");
+  check_flat(mask, at::kLong, seq.numel(), next, "mask");
+  check_flat(col, at::kLong, 1, next, "col");
+  check_flat(rng, at::kLong, 2, next, "rng");
+  c10::hip::HIPGuardMasqueradingAsCUDA g(next.device());
+  launch_token_step(next.data_ptr<int64_t>(), finished.data_ptr<bool>(), tok.data_ptr<int64_t>(),
+                    seq.data_ptr<int64_t>(), mask.data_ptr<int64_t>(), seq.size(1), seq.size(1),
+                    col.data_ptr<int64_t>(), rng.data_ptr<int64_t>(), eos, pad, (int)B, cur_stream(next));
+}
+
+void kv_advance(at::Tensor slot, at::Tensor len, at::Tensor pos) {
+  TORCH_CHECK(pos.numel() < (1ll << 31), "kv_advance: rows");
+  check_flat(pos, at::kInt, pos.numel(), pos, "pos");
+  check_flat(slot, at::kLong, 1, pos, "slot");
+  check_flat(len, at::kInt, 1, pos, "len");
+  c10::hip::HIPGuardMasqueradingAsCUDA g(pos.device());
+  launch_kv_advance(slot.data_ptr<int64_t>(), len.data_ptr<int>(), pos.data_ptr<int>(), (int)pos.numel(),
+                    cur_stream(pos));
+}
+
 }  // namespace dla
 
 TORCH_LIBRARY_FRAGMENT(dla, m) {
@@ -731,6 +769,8 @@ TORCH_LIBRARY_FRAGMENT(dla, m) {
   m.def("rope_cache_write(Tensor qkv, Tensor cos, Tensor sin, Tensor pos, Tensor(a!) k_cache, Tensor(b!) v_cache, Tensor slot, int Hq, int Hkv, int D, int rot) -> Tensor");
   m.def("decode_attn_rope(Tensor qkv, Tensor cos, Tensor sin, Tensor pos, Tensor(a!) k_cache, Tensor(b!) v_cache, Tensor slot, Tensor kv_len, Tensor? kv_start, int window, float scale, int Hq, int Hkv, int D, int rot) -> Tensor");
   m.def("sample_tokens(Tensor logits, float temperature, int top_k, float top_p, bool greedy, Tensor rng) -> Tensor");
+  m.def("token_step(Tensor next, Tensor(a!) finished, Tensor(b!) tok, Tensor(c!) seq, Tensor(d!) mask, Tensor(e!) col, Tensor(f!) rng, int eos, int pad) -> ()");
+  m.def("kv_advance(Tensor(a!) slot, Tensor(b!) len, Tensor(c!) pos) -> ()");
   m.def("skinny_gemm(Tensor x, Tensor w, Tensor(a!) counters, bool swiglu, bool glu_out=False) -> Tensor");
   m.def("skinny_glu_ks(Tensor x, Tensor w) -> Tensor");
   m.def("skinny_fused(Tensor x, Tensor w, Tensor? res, Tensor? ssq_in, float eps, bool glu) -> (Tensor, Tensor)");
@@ -746,6 +786,8 @@ TORCH_LIBRARY_FRAGMENT(dla, m) {
 TORCH_LIBRARY_IMPL(dla, CUDA, m) {
   m.impl("decode_attn", &dla::decode_attn);
   m.impl("sample_tokens", &dla::sample_tokens);
+  m.impl("token_step", &dla::token_step);
+  m.impl("kv_advance", &dla::kv_advance);
   m.impl("rope_cache_write", &dla::rope_cache_write);
   m.impl("decode_attn_rope", &dla::decode_attn_rope);
   m.impl("skinny_gemm", &dla::skinny_gemm);

@@ -323,15 +323,18 @@ __global__ __launch_bounds__(kSampNT) void sample_kernel(const T* __restrict__ l
 // Row-split sampler (plain / top-k / top-p draws) for large vocabularies. The single-block kernel above keeps
 // 8 of 256 CUs busy at B = 8 and spends ~90 us per histogram pass. Here every row is cut into G
 // chunks (G = 32 for V = 128256 -> B * 32 workgroups) and each pass is a separate launch:
-//   max     (B x G)  chunk max / argmax -> partials
-//   hist    (B x G)  chunk histogram in LDS over the pass's [lo, lo + w), z >= floor; occupied
-//                    bins added to the row histogram with global integer atomics (masses in
-//                    2^-40 fixed point, so the sums do not depend on workgroup order)
-//   resolve (B)      read + re-zero the row histogram, suffix scan, the same bin searches as
-//                    sample_kernel; writes the next pass's window / tau
-//   mass    (B x G)  kept mass of each chunk (z >= tau)
-//   pick    (B)      u ~ U(0, total) with the same Philox stream, chunk by prefix, token by a
-//                    block scan inside the chunk
+//   max   (B x G)  chunk max / argmax -> partials
+//   hist  (B x G)  chunk histogram in LDS over the pass's [lo, lo + w), z >= floor; occupied
+//                  bins added to the row histogram with global integer atomics (masses in
+//                  2^-40 fixed point, so the sums do not depend on workgroup order). The row's last workgroup
+//                  to arrive reads + re-zeroes the row histogram, takes its suffix sums and the same bin searches
+//                  as sample_kernel, and writes the next pass's window / tau
+//   mass  (B x G)  kept mass of each chunk (z >= tau). The row's last workgroup draws u ~ U(0, total) with the
+//                  same Philox stream: chunk by prefix, token by a block scan inside the chunk
+// A launch in a replayed graph costs at least 2 us whatever it does, so what one workgroup per row does (search,
+// draw) rides on the pass before it: no workgroup waits for another, the last one finds out by a counter. Top-p
+// over 16 rows of 128256: 39 us of kernels in four launches, against 42 in seven with kernels of their own for the
+// rows' searches and draws.
 // Launch count is fixed by (top_k > 0, top_p < 1), so the sequence is hipGraph-capturable; rows
 // whose thresholds settle early skip the remaining passes on the device.
 constexpr int kSplitNT = 256;
@@ -350,7 +353,9 @@ struct SplitWs {
   unsigned long long* hm;  // [B, kBins] row histogram masses, 2^-40 fixed point
   SplitState* state;  // [B]
   float* cmass;       // [B, G]
+  unsigned* tick;     // [B, kSplitTicks] workgroups arrived at each pass (the last of them: the draw)
 };
+constexpr int kSplitTicks = 8;
 
 constexpr double kFix = 1099511627776.0;  // 2^40: integer mass sums are order-independent
 
@@ -366,12 +371,13 @@ __host__ __device__ inline SplitWs split_ws(void* base, int64_t B, int G) {
   w.hm = reinterpret_cast<unsigned long long*>(p); p += align256(size_t(B) * kBins * 8);
   w.state = reinterpret_cast<SplitState*>(p); p += align256(size_t(B) * sizeof(SplitState));
   w.cmass = reinterpret_cast<float*>(p); p += align256(bg * 4);
+  w.tick = reinterpret_cast<unsigned*>(p); p += align256(size_t(B) * kSplitTicks * 4);
   return w;
 }
 inline size_t split_ws_bytes(int64_t B, int G) {
   const size_t bg = size_t(B) * G;
   return align256(bg * 4) * 3 + align256(size_t(B) * kBins * 4) + align256(size_t(B) * kBins * 8) +
-         align256(size_t(B) * sizeof(SplitState));
+         align256(size_t(B) * sizeof(SplitState)) + align256(size_t(B) * kSplitTicks * 4);
 }
 
 // chunk g of a row, in 8-element vectors: [v0, v1)
@@ -411,6 +417,7 @@ __global__ __launch_bounds__(kSplitNT) void split_max_kernel(const T* __restrict
     ws.hc[int64_t(r) * kBins + i] = 0;  // the first histogram pass accumulates into zeros
     ws.hm[int64_t(r) * kBins + i] = 0ull;
   }
+  if (g == 0 && tid < kSplitTicks) ws.tick[r * kSplitTicks + tid] = 0u;
   const T* row = logits + int64_t(r) * ld_;
   int v0, v1;
   chunk_range(V, G, g, v0, v1);
@@ -451,21 +458,100 @@ __global__ __launch_bounds__(kSplitNT) void split_max_kernel(const T* __restrict
   }
 }
 
+// True in the workgroup that arrives last (of `n`) at `tick`, for all its threads. What the others published before
+// (device-scope atomics and stores, all done when they arrive) is there for its device-scope loads, which pass the
+// caches: no cache has to be emptied.
+__device__ __forceinline__ bool split_last(unsigned* tick, int n) {
+  __shared__ bool last_s;
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    const unsigned old = __hip_atomic_fetch_add(tick, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    last_s = old == static_cast<unsigned>(n - 1);
+  }
+  __syncthreads();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+  return last_s;
+}
+
+// suffix_scan with kSplitNT threads, each in the place of kSampNT / kSplitNT of its threads: the same additions in
+// the same order (the sums are the same floats), the two copies of the running sums taking turns
+__device__ __forceinline__ void split_suffix_scan(int* c, float* m, int (*tc)[kSampNT], float (*tm)[kSampNT]) {
+  constexpr int P = kSampNT / kSplitNT;
+  int lc[P], c1[P];
+  float lm[P], m1[P];
+#pragma unroll
+  for (int p = 0; p < P; ++p) {
+    const int t = threadIdx.x + p * kSplitNT, b0 = kBins - 2 - 2 * t;
+    c1[p] = c[b0 + 1];
+    m1[p] = m[b0 + 1];
+    lc[p] = c[b0] + c1[p];
+    lm[p] = m[b0] + m1[p];
+    tc[0][t] = lc[p];
+    tm[0][t] = lm[p];
+  }
+  int k = 0;
+  for (int o = 1; o < kSampNT; o <<= 1, k ^= 1) {
+    __syncthreads();
+#pragma unroll
+    for (int p = 0; p < P; ++p) {
+      const int t = threadIdx.x + p * kSplitNT;
+      tc[k ^ 1][t] = tc[k][t] + (t >= o ? tc[k][t - o] : 0);
+      tm[k ^ 1][t] = tm[k][t] + (t >= o ? tm[k][t - o] : 0.f);
+    }
+  }
+#pragma unroll
+  for (int p = 0; p < P; ++p) {  // a thread's own places: written by itself
+    const int t = threadIdx.x + p * kSplitNT, b0 = kBins - 2 - 2 * t;
+    const int ec = tc[k][t] - lc[p];
+    const float em = tm[k][t] - lm[p];
+    c[b0 + 1] = ec + c1[p];
+    m[b0 + 1] = em + m1[p];
+    c[b0] = ec + lc[p];
+    m[b0] = em + lm[p];
+  }
+  __syncthreads();
+}
+
+// largest bin whose suffix value reaches `need` (as find_bin_*)
+template <typename V>
+__device__ __forceinline__ int split_find_bin(const V* sc, V need, int* out) {
+  if (threadIdx.x == 0) *out = 0;
+  __syncthreads();
+  for (int b = threadIdx.x; b < kBins; b += kSplitNT)
+    if (sc[b] >= need && (b == kBins - 1 || sc[b + 1] < need)) *out = b;
+  __syncthreads();
+  const int b = *out;
+  __syncthreads();
+  return b;
+}
+
 template <typename T>
 __global__ __launch_bounds__(kSplitNT) void split_hist_kernel(const T* __restrict__ logits,
                                                               int64_t ld_, int V, int G,
-                                                              float inv_t, bool first, SplitWs ws) {
+                                                              float inv_t, int pass, int top_k, float top_p,
+                                                              bool need_p, int first_phase, SplitWs ws) {
   __shared__ int c[kBins];
   __shared__ unsigned long long m[kBins];  // 2^-40 fixed point: order-independent sums
+  __shared__ int tc[2][kSampNT];
+  __shared__ float tm[2][kSampNT];
+  __shared__ int sel;
   const int r = blockIdx.y, g = blockIdx.x, tid = threadIdx.x;
-  float lo = -kRange, w = kRange, floor_z = -INFINITY;
-  if (!first) {
-    const SplitState s = ws.state[r];
+  SplitState s;
+  if (pass == 0) {  // fresh state
+    s.tau = -kRange;
+    s.lo = -kRange;
+    s.w = kRange;
+    s.floor_z = -INFINITY;
+    s.above_m = 0.f;
+    s.target = 0.f;
+    s.above_c = 0;
+    s.phase = first_phase;
+  } else {
+    s = ws.state[r];
     if (s.phase == kDone) return;
-    lo = s.lo;
-    w = s.w;
-    floor_z = s.floor_z;
   }
+  const float lo = s.lo, w = s.w, floor_z = s.floor_z;
   float gmax;
   int argmax;
   row_max(ws.pmax + r * G, ws.parg + r * G, G, gmax, argmax);
@@ -500,42 +586,32 @@ __global__ __launch_bounds__(kSplitNT) void split_hist_kernel(const T* __restric
       atomicAdd(oc + i, c[i]);
       atomicAdd(om + i, m[i]);  // same 2^-40 scale as kFix
     }
-}
+  if (!split_last(ws.tick + r * kSplitTicks + pass, G)) return;
 
-__global__ __launch_bounds__(kSampNT) void split_resolve_kernel(int G, int top_k, float top_p,
-                                                                bool need_p, int first_phase,
-                                                                SplitWs ws) {
-  __shared__ int hc[kBins];
-  __shared__ float hm[kBins];
-  __shared__ int tc[kSampNT];
-  __shared__ float tm[kSampNT];
-  __shared__ int sel;
-  const int r = blockIdx.x, tid = threadIdx.x;
-  SplitState s;
-  if (first_phase != kDone) {  // first pass: fresh state
-    s.tau = -kRange;
-    s.lo = -kRange;
-    s.w = kRange;
-    s.floor_z = -INFINITY;
-    s.above_m = 0.f;
-    s.target = 0.f;
-    s.above_c = 0;
-    s.phase = first_phase;
-  } else {
-    s = ws.state[r];
-    if (s.phase == kDone) return;
+  // ---- the row's last workgroup: its histogram, re-zeroed for the next pass, and the search
+  int* hc = c;
+  float* hm = reinterpret_cast<float*>(m);
+  constexpr int PB = kBins / kSplitNT;
+  int bc[PB];
+  unsigned long long bm[PB];
+#pragma unroll
+  for (int p = 0; p < PB; ++p) {  // every load in flight before the first is used
+    bc[p] = __hip_atomic_load(oc + tid + p * kSplitNT, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    bm[p] = __hip_atomic_load(om + tid + p * kSplitNT, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
-  for (int b = tid; b < kBins; b += kSampNT) {  // read the row histogram, re-zero it for the next pass
-    hc[b] = ws.hc[int64_t(r) * kBins + b];
-    hm[b] = (float)((double)ws.hm[int64_t(r) * kBins + b] * (1.0 / kFix));
-    ws.hc[int64_t(r) * kBins + b] = 0;
-    ws.hm[int64_t(r) * kBins + b] = 0ull;
+#pragma unroll
+  for (int p = 0; p < PB; ++p) {
+    const int b = tid + p * kSplitNT;
+    hc[b] = bc[p];
+    hm[b] = (float)((double)bm[p] * (1.0 / kFix));
+    oc[b] = 0;
+    om[b] = 0ull;
   }
   __syncthreads();
-  suffix_scan(hc, hm, tc, tm);
+  split_suffix_scan(hc, hm, tc, tm);
   const float W = kRange / kBins;
   if (s.phase == kKCoarse) {
-    const int kbin = find_bin_count(hc, top_k, &sel);
+    const int kbin = split_find_bin(hc, top_k, &sel);
     s.above_c = kbin + 1 < kBins ? hc[kbin + 1] : 0;
     s.above_m = kbin + 1 < kBins ? hm[kbin + 1] : 0.f;
     s.lo = -kRange + kbin * W;
@@ -543,14 +619,14 @@ __global__ __launch_bounds__(kSampNT) void split_resolve_kernel(int G, int top_k
     s.floor_z = -INFINITY;
     s.phase = kKFine;
   } else if (s.phase == kKFine) {
-    const int sb = find_bin_count(hc, top_k - s.above_c, &sel);
+    const int sb = split_find_bin(hc, top_k - s.above_c, &sel);
     s.tau = s.lo + sb * (W / kBins);
     const float total = s.above_m + hm[sb];
     s.phase = kDone;
     if (need_p) {
       const float target = top_p * total;
       if (s.above_m < target) {  // nucleus edge inside this same coarse bin
-        const int sp = find_bin_mass(hm, target - s.above_m, &sel);
+        const int sp = split_find_bin(hm, target - s.above_m, &sel);
         s.tau = fmaxf(s.tau, s.lo + sp * (W / kBins));
       } else {  // edge in a higher coarse bin: coarse pass again above the top-k floor
         s.target = target;
@@ -561,72 +637,64 @@ __global__ __launch_bounds__(kSampNT) void split_resolve_kernel(int G, int top_k
       }
     }
   } else if (s.phase == kPCoarse) {
-    if (first_phase == kPCoarse) s.target = top_p * hm[0];  // no top-k: total = whole row
-    const int cb = find_bin_mass(hm, s.target, &sel);
+    if (pass == 0) s.target = top_p * hm[0];  // no top-k: total = whole row
+    const int cb = split_find_bin(hm, s.target, &sel);
     s.above_m = cb + 1 < kBins ? hm[cb + 1] : 0.f;
     s.lo = -kRange + cb * W;
     s.w = W;
     s.floor_z = s.tau;
     s.phase = kPFine;
   } else {  // kPFine
-    const int sp = find_bin_mass(hm, s.target - s.above_m, &sel);
+    const int sp = split_find_bin(hm, s.target - s.above_m, &sel);
     s.tau = fmaxf(s.tau, s.lo + sp * (W / kBins));
     s.phase = kDone;
   }
-  __syncthreads();
   if (tid == 0) ws.state[r] = s;
 }
 
 template <typename T>
-__global__ __launch_bounds__(kSplitNT) void split_mass_kernel(const T* __restrict__ logits,
+__global__ __launch_bounds__(kSplitNT) void split_draw_kernel(const T* __restrict__ logits,
                                                               int64_t ld_, int V, int G,
                                                               float inv_t, bool has_tau,
-                                                              SplitWs ws) {
+                                                              const int64_t* __restrict__ rng,
+                                                              SplitWs ws,
+                                                              int64_t* __restrict__ out) {
   __shared__ float red[kSplitNT / 64];
-  const int r = blockIdx.y, g = blockIdx.x, tid = threadIdx.x;
+  __shared__ float tm[kSplitNT];
+  __shared__ int ans;
+  const int r = blockIdx.y, tid = threadIdx.x;
   float gmax;
   int argmax;
   row_max(ws.pmax + r * G, ws.parg + r * G, G, gmax, argmax);
   const float tau = has_tau ? ws.state[r].tau : -kRange;
+  const uint64_t seed = (uint64_t)rng[0], draw = (uint64_t)rng[1];
   const T* row = logits + int64_t(r) * ld_;
   int v0, v1;
-  chunk_range(V, G, g, v0, v1);
-  float acc = 0.f;
+  chunk_range(V, G, blockIdx.x, v0, v1);
+  float part = 0.f;
   for (int i = v0 + tid; i < v1; i += kSplitNT) {
     float x[8];
     ld8(row, i, x);
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
       const float z = (x[j] - gmax) * inv_t;
-      acc += z >= tau ? __expf(z) : 0.f;
+      part += z >= tau ? __expf(z) : 0.f;
     }
   }
-  const float tot = block_sum<kSplitNT>(acc, red);
-  if (tid == 0) ws.cmass[r * G + g] = tot;
-}
+  const float tot = block_sum<kSplitNT>(part, red);
+  if (tid == 0)
+    __hip_atomic_store(ws.cmass + r * G + blockIdx.x, tot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if (!split_last(ws.tick + r * kSplitTicks + kSplitTicks - 1, G)) return;
 
-template <typename T>
-__global__ __launch_bounds__(kSplitNT) void split_pick_kernel(const T* __restrict__ logits,
-                                                              int64_t ld_, int V, int G,
-                                                              float inv_t, bool has_tau,
-                                                              const int64_t* __restrict__ rng,
-                                                              SplitWs ws,
-                                                              int64_t* __restrict__ out) {
-  __shared__ float tm[kSplitNT];
-  __shared__ int ans;
-  const int r = blockIdx.x, tid = threadIdx.x;
-  float gmax;
-  int argmax;
-  row_max(ws.pmax + r * G, ws.parg + r * G, G, gmax, argmax);
-  const float tau = has_tau ? ws.state[r].tau : -kRange;
+  // ---- the row's last workgroup: the draw
   float cms[kSplitG];
+#pragma unroll
+  for (int g = 0; g < kSplitG; ++g)
+    cms[g] = __hip_atomic_load(ws.cmass + r * G + g, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   float total = 0.f;
 #pragma unroll
-  for (int g = 0; g < kSplitG; ++g) {
-    cms[g] = ws.cmass[r * kSplitG + g];
-    total += cms[g];
-  }
-  const float u = philox_uniform((uint64_t)rng[0], (uint64_t)r, (uint64_t)rng[1]) * total;
+  for (int g = 0; g < kSplitG; ++g) total += cms[g];
+  const float u = philox_uniform(seed, (uint64_t)r, draw) * total;
   // chunk holding u (every lane walks the G partials in the same order)
   int cg = -1;
   float base = 0.f, acc = 0.f;
@@ -645,18 +713,26 @@ __global__ __launch_bounds__(kSplitNT) void split_pick_kernel(const T* __restric
     acc += cm;
   }
   if (tid == 0) ans = -1;
-  const T* row = logits + int64_t(r) * ld_;
   float mine = 0.f;
   int s0 = 0, s1 = 0;
   if (cg >= 0) {
-    int v0, v1;
     chunk_range(V, G, cg, v0, v1);
     const int n = (v1 - v0) * 8, per = (n + kSplitNT - 1) / kSplitNT;
     s0 = min(n, tid * per) + v0 * 8;
     s1 = min(n, tid * per + per) + v0 * 8;
-    for (int v = s0; v < s1; ++v) {
-      const float z = (ld(row, v) - gmax) * inv_t;
+    auto add = [&](float x) {
+      const float z = (x - gmax) * inv_t;
       mine += z >= tau ? __expf(z) : 0.f;
+    };
+    if (per % 8 == 0) {  // (n is a multiple of 8: so are s0 and s1)
+      for (int v = s0; v < s1; v += 8) {
+        float x[8];
+        ld8(row, v / 8, x);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) add(x[j]);
+      }
+    } else {
+      for (int v = s0; v < s1; ++v) add(ld(row, v));
     }
   }
   tm[tid] = mine;
@@ -712,13 +788,10 @@ static void launch_split(const T* lg, int64_t ld_, int64_t rows, int V, int G, f
   const bool need_k = top_k > 0 && top_k < V, need_p = top_p < 1.f;
   split_max_kernel<T><<<grid, kSplitNT, 0, st>>>(lg, ld_, V, G, ws);
   const int passes = (need_k ? 2 : 0) + (need_p ? 2 : 0);
-  for (int p = 0; p < passes; ++p) {
-    split_hist_kernel<T><<<grid, kSplitNT, 0, st>>>(lg, ld_, V, G, inv_t, p == 0, ws);
-    const int first_phase = p == 0 ? (need_k ? kKCoarse : kPCoarse) : kDone;
-    split_resolve_kernel<<<rows, kSampNT, 0, st>>>(G, top_k, top_p, need_p, first_phase, ws);
-  }
-  split_mass_kernel<T><<<grid, kSplitNT, 0, st>>>(lg, ld_, V, G, inv_t, passes > 0, ws);
-  split_pick_kernel<T><<<rows, kSplitNT, 0, st>>>(lg, ld_, V, G, inv_t, passes > 0, rng, ws, out);
+  for (int p = 0; p < passes; ++p)
+    split_hist_kernel<T><<<grid, kSplitNT, 0, st>>>(lg, ld_, V, G, inv_t, p, top_k, top_p, need_p,
+                                                    need_k ? kKCoarse : kPCoarse, ws);
+  split_draw_kernel<T><<<grid, kSplitNT, 0, st>>>(lg, ld_, V, G, inv_t, passes > 0, rng, ws, out);
 }
 
 void launch_sample_split(const void* logits, bool is_bf16, int64_t ld_, int64_t rows, int V,
@@ -750,6 +823,53 @@ void launch_sample(const void* logits, bool is_bf16, int64_t ld_, int64_t rows, 
     else DLA_SAMPLE(float, false);
   }
 #undef DLA_SAMPLE
+}
+
+// What follows a draw in a captured token step: finished rows take the pad token, the token and its mask go to
+// column `col` of the sequence buffers and to the next step's input, rows that drew `eos` finish, and the column and
+// the draw counter advance. One workgroup does it for all rows instead of eleven launches over a few bytes each: with
+// kv_advance (one for three) and the draw's three fewer, a step of 16 rows takes 29 us less of 820.
+__global__ __launch_bounds__(256) void token_step_kernel(const int64_t* __restrict__ next, bool* __restrict__ finished,
+                                                         int64_t* __restrict__ tok, int64_t* __restrict__ seq,
+                                                         int64_t* __restrict__ mask, int64_t ld, int64_t cols,
+                                                         int64_t* __restrict__ col, int64_t* __restrict__ rng,
+                                                         int64_t eos, int64_t pad, int rows) {
+  const int64_t c = col[0], draw = rng[1];
+  for (int r = threadIdx.x; r < rows; r += 256) {
+    const bool done = finished[r];
+    const int64_t t = done ? pad : next[r];
+    if (c >= 0 && c < cols) {
+      seq[r * ld + c] = t;
+      mask[r * ld + c] = done ? 0 : 1;
+    }
+    tok[r] = t;
+    finished[r] = done || t == eos;
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    col[0] = c + 1;
+    rng[1] = draw + 1;
+  }
+}
+
+void launch_token_step(const int64_t* next, bool* finished, int64_t* tok, int64_t* seq, int64_t* mask, int64_t ld,
+                       int64_t cols, int64_t* col, int64_t* rng, int64_t eos, int64_t pad, int rows, hipStream_t st) {
+  token_step_kernel<<<1, 256, 0, st>>>(next, finished, tok, seq, mask, ld, cols, col, rng, eos, pad, rows);
+}
+
+// the device-side cache position of a captured step, one token on: three additions in one launch
+__global__ __launch_bounds__(256) void kv_advance_kernel(int64_t* __restrict__ slot, int* __restrict__ len,
+                                                         int* __restrict__ pos, int rows) {
+  const int r = blockIdx.x * 256 + threadIdx.x;
+  if (r < rows) pos[r] += 1;
+  if (r == 0) {
+    slot[0] += 1;
+    len[0] += 1;
+  }
+}
+
+void launch_kv_advance(int64_t* slot, int* len, int* pos, int rows, hipStream_t st) {
+  kv_advance_kernel<<<std::max(1, (rows + 255) / 256), 256, 0, st>>>(slot, len, pos, rows);
 }
 
 }  // namespace dla

@@ -189,9 +189,7 @@ class KVCache:
 
     def advance_device(self):
         """Device-only advance for a captured decode step (host `len` is tracked by the caller)."""
-        self.slot.add_(1)
-        self.kv_len.add_(1)
-        self.pos.add_(1)
+        ops.decode.kv_advance(self.slot, self.kv_len, self.pos)
 
 
 @dataclass
@@ -264,13 +262,8 @@ class _DecodeGraph:
     def sample(self, logits):
         t, k, p, g = self.args
         nxt = ops.decode.sample_tokens(logits, t, k, p, g, self.rng)
-        nxt = torch.where(self.finished, torch.full_like(nxt, self.pad), nxt)
-        self.gen_mask.index_copy_(1, self.col, (~self.finished).long().unsqueeze(1))
-        self.out.index_copy_(1, self.col, nxt.unsqueeze(1))
-        self.finished |= nxt == self.eos
-        self.tok.copy_(nxt.unsqueeze(1))
-        self.col.add_(1)
-        self.rng[1:].add_(1)
+        ops.decode.token_step(nxt, self.finished, self.tok, self.out, self.gen_mask, self.col, self.rng, self.eos,
+                              self.pad)
 
     def reset(self, seed: int):
         self.tok.zero_()

@@ -62,6 +62,32 @@ def sample_tokens(logits: torch.Tensor, temperature: float, top_k: int, top_p: f
     return sample_next(logits.float(), not greedy, temperature, top_p, top_k, generator)
 
 
+def kv_advance(slot: torch.Tensor, kv_len: torch.Tensor, pos: torch.Tensor) -> None:
+    """The cache position held on the device, one token on (in place)."""
+    if _ext.use_native(pos):
+        _ext.require().kv_advance(slot, kv_len, pos)
+    else:
+        for t in (slot, kv_len, pos):
+            t.add_(1)
+
+
+def token_step(nxt: torch.Tensor, finished: torch.Tensor, tok: torch.Tensor, seq: torch.Tensor, mask: torch.Tensor,
+               col: torch.Tensor, rng: torch.Tensor, eos: Optional[int], pad: int) -> None:
+    """Bookkeeping of one drawn token per row, in place: finished rows take `pad`, column `col` of `seq` and `mask` (1 where
+    the row was not finished) and the next input `tok` are written, rows that drew `eos` finish, `col` and the draw
+    counter rng[1] advance."""
+    if _ext.use_native(nxt):
+        _ext.require().token_step(nxt, finished, tok, seq, mask, col, rng, -1 if eos is None else int(eos), int(pad))
+        return
+    nxt = torch.where(finished, torch.full_like(nxt, pad), nxt)
+    mask.index_copy_(1, col, (~finished).long().unsqueeze(1))
+    seq.index_copy_(1, col, nxt.unsqueeze(1))
+    finished |= nxt == eos
+    tok.copy_(nxt.unsqueeze(1))
+    col.add_(1)
+    rng[1:].add_(1)
+
+
 # ------------------------------------------------------------------------- skinny GEMM (M <= 16)
 SKINNY = os.environ.get("DLA_SKINNY", "1") != "0"
 # Every decode GEMM takes the skinny kernels: wide outputs (>= 128 column blocks) the LDS-staged
