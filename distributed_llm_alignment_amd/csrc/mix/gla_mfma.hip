@@ -138,6 +138,15 @@ __device__ __forceinline__ bf16x8 value8(const GlaParams& p, const Head& x, int 
   return r;
 }
 
+// 8 fp32 values into the hi and lo planes of an image
+template <int N>
+__device__ __forceinline__ void put_row(bf16_t (*img)[N], int at, const float* v) {
+  s16x8 hi, lo;
+  Mma<bf16_t>::split(v, hi, lo);
+  store_bf16x8(&img[0][at], __builtin_bit_cast(bf16x8, hi));
+  store_bf16x8(&img[1][at], __builtin_bit_cast(bf16x8, lo));
+}
+
 // grid (nc * ceil(vdim / 128), H, B): wave w = value rows 32 w .. + 31 of the block, all of dim
 template <int ND>
 __global__ __launch_bounds__(kThreads, ND > 4 ? 1 : 2) void gla_state_kernel(GlaParams p) {
@@ -237,6 +246,7 @@ __global__ __launch_bounds__(256) void gla_scan_kernel(GlaParams p) {
 template <int NK, int NV>
 __global__ __launch_bounds__(kThreads, NK > 8 || NV > 4 ? 1 : 2) void gla_output_kernel(GlaParams p) {
   constexpr int DW = 16 * NK, SK = row_stride(DW), SV = tr_stride(32 * NV), CK = 2 * NK, CV = 4 * NV;
+  constexpr int LK = kBN * CK / kThreads;  // 8-wide pieces of a key image per thread
   __shared__ __attribute__((aligned(16))) bf16_t ks[2][kBN * SK];
   __shared__ __attribute__((aligned(16))) bf16_t vs[kBN * SV];
   __shared__ float sub[4][DW];   // log2 total of each sub-chunk
@@ -266,20 +276,35 @@ __global__ __launch_bounds__(kThreads, NK > 8 || NV > 4 ? 1 : 2) void gla_output
     fac[6][d] = exp2f(e[2]);
     if (!ok) fast = 0;
   }
-  // q 2^(l_t) as planes
+  // q 2^(l_t) as planes. Queries and the state's rows come through the key image (64 rows), read from memory a row
+  // at a time and split once for all waves; read as operands by every wave (a row per lane, 16 bytes of 64 rows per
+  // instruction) they kept the address path busy: 116 us for 5000 tokens of 16 heads of 128, 85 so.
   s16x8 qh[NK], ql[NK];
 #pragma unroll
-  for (int s = 0; s < NK; ++s) {
-    const int d = 16 * s + 8 * g;
-    float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    if (tq < x.len && d < p.dim) {
-      float l[8];
-      load_vec<bf16_t, 8>(x.in + tq * p.ld + x.h * p.dim + d, v);
-      load_vec<float, 8>(x.cum + static_cast<int64_t>(tq) * x.Hd + d, l);
+  for (int half = 0; half < 2; ++half) {
+    if (half) __syncthreads();
 #pragma unroll
-      for (int e = 0; e < 8; ++e) v[e] *= p.qscale * __builtin_amdgcn_exp2f(l[e]);
+    for (int j = 0; j < LK; ++j) {
+      const int i = threadIdx.x + kThreads * j, r = i / CK, t = half * kBN + r, d = (i % CK) * 8;
+      float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+      if (t < x.len && d < p.dim) {
+        float l[8];
+        load_vec<bf16_t, 8>(x.in + t * p.ld + x.h * p.dim + d, v);
+        load_vec<float, 8>(x.cum + static_cast<int64_t>(t) * x.Hd + d, l);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[e] *= p.qscale * __builtin_amdgcn_exp2f(l[e]);
+      }
+      put_row(ks, r * SK + d, v);
     }
-    Mma<bf16_t>::split(v, qh[s], ql[s]);
+    __syncthreads();
+    if (wave >> 1 == half) {
+#pragma unroll
+      for (int s = 0; s < NK; ++s) {
+        const int at = ((wave & 1) * 32 + c32) * SK + 16 * s + 8 * g;
+        qh[s] = __builtin_bit_cast(s16x8, load_bf16x8(&ks[0][at]));
+        ql[s] = __builtin_bit_cast(s16x8, load_bf16x8(&ks[1][at]));
+      }
+    }
   }
   // step s of the query times factor row f
   auto scaled = [&](int s, const float* f, s16x8& h, s16x8& l) {
@@ -294,24 +319,38 @@ __global__ __launch_bounds__(kThreads, NK > 8 || NV > 4 ? 1 : 2) void gla_output
   for (int t = 0; t < NV; ++t)
 #pragma unroll
     for (int i = 0; i < 16; ++i) o[t][i] = 0.f;
-  __syncthreads();
   if (!p.fresh || blockIdx.x > 0) {  // (chunk 0 of a fresh sequence starts at zero)
     const float* S = p.work + ((static_cast<int64_t>(x.b) * p.H + x.h) * p.nc + blockIdx.x) * p.vdim * p.dim;
 #pragma unroll
-    for (int s = 0; s < NK; ++s) {
-      const int d = 16 * s + 8 * g;
-      s16x8 ah, al;
-      scaled(s, fac[wave], ah, al);
+    for (int v0 = 0; v0 < 32 * NV; v0 += kBN) {
+      float y[LK][8];
 #pragma unroll
-      for (int t = 0; t < NV; ++t) {
-        const int v = 32 * t + c32;
-        float y[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-        if (d < p.dim && v < p.vdim) load_vec<float, 8>(S + static_cast<int64_t>(v) * p.dim + d, y);
-        s16x8 sh, sl;
-        Mma<bf16_t>::split(y, sh, sl);
-        o[t] = mfma32(sh, ah, o[t]);
-        o[t] = mfma32(sl, ah, o[t]);
-        o[t] = mfma32(sh, al, o[t]);
+      for (int j = 0; j < LK; ++j) {
+        const int i = threadIdx.x + kThreads * j, v = v0 + i / CK, d = (i % CK) * 8;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) y[j][e] = 0.f;
+        if (d < p.dim && v < p.vdim) load_vec<float, 8>(S + static_cast<int64_t>(v) * p.dim + d, y[j]);
+      }
+      __syncthreads();
+#pragma unroll
+      for (int j = 0; j < LK; ++j) {
+        const int i = threadIdx.x + kThreads * j;
+        put_row(ks, (i / CK) * SK + (i % CK) * 8, y[j]);
+      }
+      __syncthreads();
+#pragma unroll
+      for (int s = 0; s < NK; ++s) {
+        s16x8 ah, al;
+        scaled(s, fac[wave], ah, al);
+#pragma unroll
+        for (int n = 0; n < 2; ++n) {
+          f32x16& ot = o[v0 / 32 + n];
+          const s16x8 sh = __builtin_bit_cast(s16x8, load_bf16x8(&ks[0][(32 * n + c32) * SK + 16 * s + 8 * g]));
+          const s16x8 sl = __builtin_bit_cast(s16x8, load_bf16x8(&ks[1][(32 * n + c32) * SK + 16 * s + 8 * g]));
+          ot = mfma32(sh, ah, ot);
+          ot = mfma32(sl, ah, ot);
+          ot = mfma32(sh, al, ot);
+        }
       }
     }
   }
@@ -393,27 +432,41 @@ __global__ __launch_bounds__(kThreads, NK > 8 || NV > 4 ? 1 : 2) void gla_output
 #pragma unroll
     for (int i = 0; i < 16; ++i) ss += o[t][i] * o[t][i];  // (rows past vdim are zero)
   ss += __shfl_xor(ss, 32, 64);
-  if (tq >= x.len) return;
   const float rs = rsqrtf(ss / p.vdim + p.eps);
-  const bf16_t* gr = x.in + tq * p.ld + 2 * x.Hd + Hv + x.h * p.vdim;
+  // out through the wave's part of the key image, EW columns at a time: gates and outputs move whole rows
+  constexpr int EW = sizeof(ks) >= 4 * 32 * (64 + 4) * sizeof(float) ? 64 : 32, SE = EW + 4, CE = EW / 8;
+  static_assert(sizeof(ks) >= 4 * 32 * SE * sizeof(float) && 32 * NV % EW == 0, "exchange tile");
+  float* ex = reinterpret_cast<float*>(&ks[0][0]) + wave * 32 * SE;
   const bf16_t* nw = static_cast<const bf16_t*>(p.norm_w);
-  bf16_t* yr = static_cast<bf16_t*>(p.y) + (static_cast<int64_t>(x.b) * p.T + x.t0 + tq) * Hv + x.h * p.vdim;
+  __syncthreads();
 #pragma unroll
-  for (int t = 0; t < NV; ++t)
+  for (int v0 = 0; v0 < 32 * NV; v0 += EW) {
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      const int v = 32 * t + 8 * u + 4 * g;
-      if (v >= p.vdim) continue;
-      const bf16x4 gv = *reinterpret_cast<const bf16x4*>(gr + v), wv = *reinterpret_cast<const bf16x4*>(nw + v);
-      float y[4];
+    for (int t = 0; t < EW / 32; ++t)
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const float z = bf2f(gv[e]);
-        y[e] = o[t][4 * u + e] * rs * bf2f(wv[e]) * (z / (1.f + __expf(-z)));
+      for (int u = 0; u < 4; ++u) {
+        const f32x16& ot = o[v0 / 32 + t];
+        *reinterpret_cast<f32x4*>(ex + c32 * SE + 32 * t + 8 * u + 4 * g) =
+            f32x4{ot[4 * u] * rs, ot[4 * u + 1] * rs, ot[4 * u + 2] * rs, ot[4 * u + 3] * rs};
       }
-      typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-      *reinterpret_cast<u32x2*>(yr + v) = u32x2{pack2bf(y[0], y[1]), pack2bf(y[2], y[3])};
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int j = 0; j < 32 * CE / 64; ++j) {
+      const int i = lane + 64 * j, t = wave * 32 + i / CE, v = v0 + (i % CE) * 8;
+      if (t >= x.len || v >= p.vdim) continue;
+      const bf16x8 gv = load_bf16x8(x.in + t * p.ld + 2 * x.Hd + Hv + x.h * p.vdim + v), wv = load_bf16x8(nw + v);
+      float y[8];
+      load_vec<float, 8>(ex + (i / CE) * SE + (i % CE) * 8, y);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const float z = bf2f(gv[e]);
+        y[e] = y[e] * bf2f(wv[e]) * (z / (1.f + __expf(-z)));
+      }
+      store_bf16x8(static_cast<bf16_t*>(p.y) + (static_cast<int64_t>(x.b) * p.T + x.t0 + t) * Hv + x.h * p.vdim + v,
+                   pack_bf16x8(y));
     }
+    __builtin_amdgcn_wave_barrier();
+  }
 }
 
 }  // namespace

@@ -58,6 +58,15 @@ __device__ __forceinline__ bf16x8 value8(const RetentionParams& p, const Head& h
   return r;
 }
 
+// 8 fp32 values into the hi and lo planes of an image
+template <int N>
+__device__ __forceinline__ void put_row(bf16_t (*img)[N], int at, const float* v) {
+  s16x8 hi, lo;
+  Mma<bf16_t>::split(v, hi, lo);
+  store_bf16x8(&img[0][at], __builtin_bit_cast(bf16x8, hi));
+  store_bf16x8(&img[1][at], __builtin_bit_cast(bf16x8, lo));
+}
+
 // grid (nc * ceil(vdim / 128), H, B): wave w = value rows 32 w .. + 31 of the block, all of dim
 template <int ND>
 __global__ __launch_bounds__(kThreads, ND > 4 ? 1 : 2) void ret_state_mfma_kernel(RetentionParams p) {
@@ -122,6 +131,7 @@ __global__ __launch_bounds__(kThreads, ND > 4 ? 1 : 2) void ret_state_mfma_kerne
 template <int NK, int NV>
 __global__ __launch_bounds__(kThreads, NK > 8 ? 1 : 2) void ret_output_mfma_kernel(RetentionParams p) {
   constexpr int SK = row_stride(16 * NK), SV = tr_stride(32 * NV), CK = 2 * NK, CV = 4 * NV;
+  constexpr int LK = kBN * CK / kThreads;  // 8-wide pieces of a key image per thread
   __shared__ __attribute__((aligned(16))) bf16_t ks[2][kBN * SK];
   __shared__ __attribute__((aligned(16))) bf16_t vs[kBN * SV];
   const Head hd = head_of(p, blockIdx.y, blockIdx.z);
@@ -129,12 +139,29 @@ __global__ __launch_bounds__(kThreads, NK > 8 ? 1 : 2) void ret_output_mfma_kern
   const int Hd = p.H * p.dim, Hv = p.H * p.vdim;
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, c32 = lane & 31, g = lane >> 5;
   const int tq = wave * 32 + c32;  // this lane's token in the chunk
+  // Queries and the state's rows come through the key image (64 rows of hi and lo planes), read from memory a row
+  // at a time and split once for all waves; read as operands by every wave (a row per lane, 16 bytes of 64 rows per
+  // instruction) they kept the address path busy: 67 us for 4 x 1024 tokens of 16 heads of 128, 54 so.
   s16x8 qh[NK], ql[NK];
 #pragma unroll
-  for (int s = 0; s < NK; ++s) {
-    float v[8];
-    rotated8(p, hd, hd.h * p.dim, t0 + tq, 16 * s + 8 * g, t0 + len, false, v);
-    Mma<bf16_t>::split(v, qh[s], ql[s]);
+  for (int half = 0; half < 2; ++half) {
+    if (half) __syncthreads();
+#pragma unroll
+    for (int j = 0; j < LK; ++j) {
+      const int i = threadIdx.x + kThreads * j, t = i / CK, d = (i % CK) * 8;
+      float v[8];
+      rotated8(p, hd, hd.h * p.dim, t0 + half * kBN + t, d, t0 + len, false, v);
+      put_row(ks, t * SK + d, v);
+    }
+    __syncthreads();
+    if (wave >> 1 == half) {
+#pragma unroll
+      for (int s = 0; s < NK; ++s) {
+        const int at = ((wave & 1) * 32 + c32) * SK + 16 * s + 8 * g;
+        qh[s] = __builtin_bit_cast(s16x8, load_bf16x8(&ks[0][at]));
+        ql[s] = __builtin_bit_cast(s16x8, load_bf16x8(&ks[1][at]));
+      }
+    }
   }
   f32x16 o[NV];
 #pragma unroll
@@ -145,22 +172,36 @@ __global__ __launch_bounds__(kThreads, NK > 8 ? 1 : 2) void ret_output_mfma_kern
     const float* S = p.work + ((static_cast<int64_t>(hd.b) * p.H + hd.h) * p.nc + blockIdx.x) * p.vdim * p.dim;
     const float f = exp2f(static_cast<float>(tq + 1) * hd.l2);
 #pragma unroll
-    for (int t = 0; t < NV; ++t) {
-      const int v = 32 * t + c32;
-      const float* row = S + static_cast<int64_t>(min(v, p.vdim - 1)) * p.dim;
+    for (int v0 = 0; v0 < 32 * NV; v0 += kBN) {
+      float x[LK][8];
 #pragma unroll
-      for (int s = 0; s < NK; ++s) {
-        const int d = 16 * s + 8 * g;
-        float x[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-        if (d < p.dim && v < p.vdim) load_vec<float, 8>(row + d, x);
-        s16x8 sh, sl;
-        Mma<bf16_t>::split(x, sh, sl);
-        o[t] = mfma32(sh, qh[s], o[t]);
-        o[t] = mfma32(sl, qh[s], o[t]);
-        o[t] = mfma32(sh, ql[s], o[t]);
+      for (int j = 0; j < LK; ++j) {
+        const int i = threadIdx.x + kThreads * j, v = v0 + i / CK, d = (i % CK) * 8;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) x[j][e] = 0.f;
+        if (d < p.dim && v < p.vdim) load_vec<float, 8>(S + static_cast<int64_t>(v) * p.dim + d, x[j]);
       }
+      __syncthreads();
 #pragma unroll
-      for (int i = 0; i < 16; ++i) o[t][i] *= f;
+      for (int j = 0; j < LK; ++j) {
+        const int i = threadIdx.x + kThreads * j;
+        put_row(ks, (i / CK) * SK + (i % CK) * 8, x[j]);
+      }
+      __syncthreads();
+#pragma unroll
+      for (int n = 0; n < 2; ++n) {
+        f32x16& ot = o[v0 / 32 + n];
+#pragma unroll
+        for (int s = 0; s < NK; ++s) {
+          const s16x8 sh = __builtin_bit_cast(s16x8, load_bf16x8(&ks[0][(32 * n + c32) * SK + 16 * s + 8 * g]));
+          const s16x8 sl = __builtin_bit_cast(s16x8, load_bf16x8(&ks[1][(32 * n + c32) * SK + 16 * s + 8 * g]));
+          ot = mfma32(sh, qh[s], ot);
+          ot = mfma32(sl, qh[s], ot);
+          ot = mfma32(sh, ql[s], ot);
+        }
+#pragma unroll
+        for (int i = 0; i < 16; ++i) ot[i] *= f;
+      }
     }
   }
   for (int s0 = 0; s0 < len; s0 += kBN) {
@@ -224,27 +265,40 @@ __global__ __launch_bounds__(kThreads, NK > 8 ? 1 : 2) void ret_output_mfma_kern
 #pragma unroll
     for (int i = 0; i < 16; ++i) ss += o[t][i] * o[t][i];  // (rows past vdim are zero)
   ss += __shfl_xor(ss, 32, 64);
-  if (tq >= len) return;
   const float rs = rsqrtf(ss / p.vdim + p.eps);
-  const int64_t row = static_cast<int64_t>(hd.b) * p.T + t0 + tq;
-  const bf16_t* gr = static_cast<const bf16_t*>(p.qkvg) + row * p.ld + 2 * Hd + Hv + hd.h * p.vdim;
-  bf16_t* yr = static_cast<bf16_t*>(p.y) + row * Hv + hd.h * p.vdim;
+  // out through the wave's part of the key image, EW columns at a time: gates and outputs move whole rows
+  constexpr int EW = sizeof(ks) >= 4 * 32 * (64 + 4) * sizeof(float) ? 64 : 32, SE = EW + 4, CE = EW / 8;
+  static_assert(sizeof(ks) >= 4 * 32 * SE * sizeof(float) && 32 * NV % EW == 0, "exchange tile");
+  float* ex = reinterpret_cast<float*>(&ks[0][0]) + wave * 32 * SE;
+  __syncthreads();
 #pragma unroll
-  for (int t = 0; t < NV; ++t)
+  for (int v0 = 0; v0 < 32 * NV; v0 += EW) {
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      const int v = 32 * t + 8 * u + 4 * g;
-      if (v >= p.vdim) continue;
-      const bf16x4 gv = *reinterpret_cast<const bf16x4*>(gr + v);
-      float y[4];
+    for (int t = 0; t < EW / 32; ++t)
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const float z = bf2f(gv[e]);
-        y[e] = o[t][4 * u + e] * rs * (z / (1.f + __expf(-z)));
+      for (int u = 0; u < 4; ++u) {
+        const f32x16& ot = o[v0 / 32 + t];
+        *reinterpret_cast<f32x4*>(ex + c32 * SE + 32 * t + 8 * u + 4 * g) =
+            f32x4{ot[4 * u] * rs, ot[4 * u + 1] * rs, ot[4 * u + 2] * rs, ot[4 * u + 3] * rs};
       }
-      typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-      *reinterpret_cast<u32x2*>(yr + v) = u32x2{pack2bf(y[0], y[1]), pack2bf(y[2], y[3])};
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int j = 0; j < 32 * CE / 64; ++j) {
+      const int i = lane + 64 * j, r = i / CE, v = v0 + (i % CE) * 8;
+      if (wave * 32 + r >= len || v >= p.vdim) continue;
+      const int64_t row = static_cast<int64_t>(hd.b) * p.T + t0 + wave * 32 + r;
+      const bf16x8 gv = load_bf16x8(static_cast<const bf16_t*>(p.qkvg) + row * p.ld + 2 * Hd + Hv + hd.h * p.vdim + v);
+      float y[8];
+      load_vec<float, 8>(ex + r * SE + (i % CE) * 8, y);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const float z = bf2f(gv[e]);
+        y[e] = y[e] * (z / (1.f + __expf(-z)));
+      }
+      store_bf16x8(static_cast<bf16_t*>(p.y) + row * Hv + hd.h * p.vdim + v, pack_bf16x8(y));
     }
+    __builtin_amdgcn_wave_barrier();
+  }
 }
 
 }  // namespace
