@@ -75,3 +75,34 @@ def test_linear_logprob_padded_rows(V):
     assert float((got.double() - lp).norm()) <= 8e-3 * float(lp.norm())
     for a, b in ((h, hd), (w, wd)):
         assert float((a.grad.double() - b.grad).norm()) <= 2e-2 * float(b.grad.norm())
+
+
+@pytest.mark.parametrize("N,H", [(1, 8), (16, 8), (17, 520), (33, 512), (4100, 768)])
+@pytest.mark.parametrize("gdtype", [torch.bfloat16, torch.float32])
+def test_embedding_runs(N, H, gdtype):
+    """Runs of every length and place (one id, no repeats, the pad id over most positions, invalid ids at both ends) into a
+    gradient that holds something already: float64 sums; fp32 over a run (n * 2^-24 relative), bf16 rounds once (2^-8)."""
+    from distributed_llm_alignment_amd.ops import _ext
+
+    V = 97
+    g0 = torch.Generator(device=DEV).manual_seed(N + H)
+    for case in range(4):
+        ids = torch.randint(0, V, (N,), generator=g0, device=DEV)
+        if case == 0:
+            ids.fill_(V - 1)
+        elif case == 1:
+            ids = torch.arange(N, device=DEV) * V // max(N, V)
+        elif case == 2:
+            ids[torch.rand(N, generator=g0, device=DEV) < 0.8] = 3
+        else:
+            ids[: N // 3] = -1
+            ids[N - N // 4:] = V
+        dy = torch.randn(N, H, generator=g0, device=DEV).bfloat16()
+        grad = torch.randn(V, H, generator=g0, device=DEV).to(gdtype)
+        ok = (ids >= 0) & (ids < V)
+        want = grad.double().index_add(0, ids[ok], dy[ok].double())
+        sid, perm = torch.sort(ids, stable=True)
+        _ext.require().embed_bwd(sid, perm, dy, grad)
+        size = grad.double().abs().index_add(0, ids[ok], dy[ok].double().abs())
+        tol = (2 ** -8 if gdtype == torch.bfloat16 else 0) * want.abs() + N * 2 ** -24 * size
+        assert bool(((grad.double() - want).abs() <= tol).all()), case
