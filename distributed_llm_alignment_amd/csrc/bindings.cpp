@@ -84,6 +84,8 @@ void launch_attn_dkv_reduce(const float*, const float*, int, int, int, int, int,
                             const float*, const float*, const int*, int, hipStream_t, const bf16_t*,
                             const bf16_t*);
 void launch_transpose_bf16(const bf16_t*, int64_t, int64_t, int64_t, bf16_t*, int64_t, hipStream_t);
+int column_sum_blocks(int64_t, int);
+void launch_column_sum(const bf16_t*, int64_t, int64_t, int, float*, bf16_t*, hipStream_t);
 
 // ================================= norms ======================================================
 std::tuple<at::Tensor, at::Tensor, at::Tensor, at::Tensor> norm_fwd(
@@ -569,6 +571,21 @@ void attn_bwd(const at::Tensor& dout, const at::Tensor& q, const at::Tensor& k,
 }
 
 // out [C, R] <- in [R, C]^T (both row-major with unit column stride, 16-byte aligned rows)
+// x [R, C] bf16 (unit column stride, 16-byte aligned rows) -> its column sums [C]
+at::Tensor column_sum(const at::Tensor& x) {
+  check_bf16(x, "x");
+  TORCH_CHECK(x.dim() == 2 && x.stride(1) == 1 && x.stride(0) % 8 == 0 && x.size(1) % 8 == 0 && x.size(0) > 0 &&
+                  x.size(1) > 0 && x.size(0) < (1ll << 31) && x.size(1) < (1ll << 31),
+              "column_sum: [R, C] with 16-byte aligned rows, C % 8 == 0");
+  check_aligned16(x, "x");
+  c10::hip::HIPGuardMasqueradingAsCUDA g(x.device());
+  const int cols = static_cast<int>(x.size(1));
+  auto part = at::empty({column_sum_blocks(x.size(0), cols), cols}, x.options().dtype(at::kFloat));
+  auto out = at::empty({cols}, x.options());
+  launch_column_sum(cbp(x), x.stride(0), x.size(0), cols, part.data_ptr<float>(), bp(out), cur_stream(x));
+  return out;
+}
+
 void transpose_bf16(const at::Tensor& in, at::Tensor& out) {
   check_bf16(in, "in");
   check_bf16(out, "out");
@@ -925,6 +942,7 @@ TORCH_LIBRARY(dla, m) {
   m.def("attn_bwd(Tensor dout, Tensor q, Tensor k, Tensor v, Tensor o, Tensor lse2, Tensor(a!) dq, Tensor(b!) dk, Tensor(c!) dv, float scale, bool causal, int causal_off, int window, Tensor? kv_start, Tensor? kv_end, Tensor? segs=None, Tensor? rope_cos=None, Tensor? rope_sin=None, Tensor? rope_pos=None, bool rope_inputs=False) -> ()");
   m.def("attn_stamps(Tensor like) -> Tensor");
   m.def("attn_fwd_switch(str name, int value) -> int", &dla::attn_fwd_switch);
+  m.def("column_sum(Tensor x) -> Tensor");
   m.def("transpose_bf16(Tensor input, Tensor(a!) out) -> ()");
   m.def("logprob_fwd(Tensor logits, Tensor targets, int vocab_offset=0) -> (Tensor, Tensor)");
   m.def("logprob_bwd(Tensor(a!) logits, Tensor targets, Tensor lse, Tensor grad, int vocab_offset=0) -> ()");
@@ -958,6 +976,7 @@ TORCH_LIBRARY_IMPL(dla, CUDA, m) {
   m.impl("attn_fwd", &dla::attn_fwd);
   m.impl("attn_bwd", &dla::attn_bwd);
   m.impl("attn_stamps", &dla::attn_stamps);
+  m.impl("column_sum", &dla::column_sum);
   m.impl("transpose_bf16", &dla::transpose_bf16);
   m.impl("logprob_fwd", &dla::logprob_fwd);
   m.impl("logprob_bwd", &dla::logprob_bwd);

@@ -317,4 +317,76 @@ void launch_gelu_bwd(const bf16_t* x, const bf16_t* dy, bf16_t* dx, int64_t n, h
   gelu_bwd_kernel<<<grid_for(n / 8), 256, 0, st>>>(x, dy, dx, n / 8);
 }
 
+// Column sums of a bf16 matrix [rows, cols] (a bias gradient): fp32 sums in a fixed order, one rounding. Read once at
+// 512 bytes per row and block; the rows are cut so that about 1024 workgroups are in flight, and a second launch adds
+// their fp32 partial sums. 8000 rows: 768 columns 5 + 6 us, 3072 columns 11 + 5, against 20 + 5 and 27 + 5 for the
+// library's reduction and the clearing of its counters.
+constexpr int kSumCols = 256, kSumStep = 8;  // columns per workgroup; rows it reads at a time (2 per wave)
+
+__global__ __launch_bounds__(256) void column_sum_kernel(const bf16_t* __restrict__ x, int64_t ld, int64_t rows, int cols,
+                                                         int per, float* __restrict__ part) {
+  __shared__ float red[kSumStep][kSumCols + 4];
+  const int sub = threadIdx.x >> 5, c = (threadIdx.x & 31) * 8, col = blockIdx.x * kSumCols + c;
+  const int64_t r0 = static_cast<int64_t>(blockIdx.y) * per, r1 = min(r0 + per, rows);
+  float a[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+  if (col < cols) {
+    const bf16_t* p = x + (r0 + sub) * ld + col;
+    constexpr int U = 4;
+    int64_t r = r0 + sub;
+    for (; r + (U - 1) * kSumStep < r1; r += U * kSumStep, p += U * kSumStep * ld) {
+      bf16x8 v[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) v[u] = load_bf16x8(p + u * kSumStep * ld);
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) a[e] += bf2f(v[u][e]);
+    }
+    for (; r < r1; r += kSumStep, p += kSumStep * ld) {
+      const bf16x8 v = load_bf16x8(p);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) a[e] += bf2f(v[e]);
+    }
+  }
+  *reinterpret_cast<f32x4*>(&red[sub][c]) = f32x4{a[0], a[1], a[2], a[3]};
+  *reinterpret_cast<f32x4*>(&red[sub][c + 4]) = f32x4{a[4], a[5], a[6], a[7]};
+  __syncthreads();
+  const int mine = blockIdx.x * kSumCols + threadIdx.x;
+  if (mine >= cols) return;
+  float t = 0.f;
+#pragma unroll
+  for (int s = 0; s < kSumStep; ++s) t += red[s][threadIdx.x];
+  part[static_cast<int64_t>(blockIdx.y) * cols + mine] = t;
+}
+
+__global__ __launch_bounds__(1024) void column_sum_fold_kernel(const float* __restrict__ part, int n, int cols,
+                                                               bf16_t* __restrict__ out) {
+  __shared__ float red[16][64];
+  const int sub = threadIdx.x >> 6, lane = threadIdx.x & 63, col = blockIdx.x * 64 + lane;
+  float t = 0.f;
+  if (col < cols) {
+#pragma unroll 16
+    for (int r = sub; r < n; r += 16) t += part[static_cast<int64_t>(r) * cols + col];
+  }
+  red[sub][lane] = t;
+  __syncthreads();
+  if (sub || col >= cols) return;
+#pragma unroll
+  for (int s = 1; s < 16; ++s) t += red[s][lane];
+  out[col] = f2bf(t);
+}
+
+// row blocks (rows of the workspace [blocks, cols])
+int column_sum_blocks(int64_t rows, int cols) {
+  const int64_t want = std::max<int64_t>(1, 1024 / ((cols + kSumCols - 1) / kSumCols));
+  return static_cast<int>(std::min(want, std::max<int64_t>(1, (rows + 4 * kSumStep - 1) / (4 * kSumStep))));
+}
+
+void launch_column_sum(const bf16_t* x, int64_t ld, int64_t rows, int cols, float* part, bf16_t* out, hipStream_t st) {
+  const int n = column_sum_blocks(rows, cols);
+  const int per = static_cast<int>(((rows + n - 1) / n + kSumStep - 1) / kSumStep * kSumStep);
+  column_sum_kernel<<<dim3((cols + kSumCols - 1) / kSumCols, n), 256, 0, st>>>(x, ld, rows, cols, per, part);
+  column_sum_fold_kernel<<<(cols + 63) / 64, 1024, 0, st>>>(part, n, cols, out);
+}
+
 }  // namespace dla

@@ -124,6 +124,15 @@ def uses_main_grad(weight: torch.Tensor) -> bool:
             and not getattr(weight, "_dla_shared", False))
 
 
+def bias_grad(dy2: torch.Tensor) -> torch.Tensor:
+    """dy2.sum(0), fp32 sums rounded once."""
+    M, N = dy2.shape
+    if (M > 0 and N > 0 and N % 8 == 0 and dy2.dtype == torch.bfloat16 and dy2.stride(1) == 1 and dy2.stride(0) % 8 == 0
+            and dy2.data_ptr() % 16 == 0 and _ext.use_native(dy2)):
+        return _ext.require().column_sum(dy2)
+    return dy2.sum(0)
+
+
 class _LinearMainGradFn(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, weight, bias):
@@ -147,7 +156,7 @@ class _LinearMainGradFn(torch.autograd.Function):
             x2 = x.reshape(-1, K)
             if not accumulate_weight_grad(weight, dy2, x2):
                 dw = dy2.t() @ x2
-        db = dy2.sum(0) if (ctx.has_bias and ctx.needs_input_grad[2]) else None
+        db = bias_grad(dy2) if (ctx.has_bias and ctx.needs_input_grad[2]) else None
         return dx, dw, db
 
 

@@ -106,3 +106,17 @@ def test_embedding_runs(N, H, gdtype):
         size = grad.double().abs().index_add(0, ids[ok], dy[ok].double().abs())
         tol = (2 ** -8 if gdtype == torch.bfloat16 else 0) * want.abs() + N * 2 ** -24 * size
         assert bool(((grad.double() - want).abs() <= tol).all()), case
+
+
+@pytest.mark.parametrize("M,N,pad", [(1, 8, 0), (7, 256, 0), (33, 264, 8), (1000, 768, 0), (8000, 2304, 0), (4097, 3072, 16)])
+def test_column_sum(M, N, pad):
+    """Bias gradients over row and column remainders and a padded stride, against float64: fp32 sums (M * 2^-24 of the sum of
+    sizes at most) and one bf16 rounding; a stride the kernel does not take gives the same."""
+    from distributed_llm_alignment_amd.ops.linear import bias_grad
+
+    g0 = torch.Generator(device=DEV).manual_seed(M + N)
+    x = torch.randn(M, N + pad, generator=g0, device=DEV).bfloat16()[:, :N]
+    want, size = x.double().sum(0), x.double().abs().sum(0)
+    odd = torch.empty(M, N + pad + 1, dtype=x.dtype, device=DEV)[:, :N].copy_(x)
+    for y in (x, odd):
+        assert bool(((bias_grad(y).double() - want).abs() <= 2 ** -8 * want.abs() + M * 2 ** -24 * size).all())
