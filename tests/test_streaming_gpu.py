@@ -120,3 +120,32 @@ def test_column_sum(M, N, pad):
     odd = torch.empty(M, N + pad + 1, dtype=x.dtype, device=DEV)[:, :N].copy_(x)
     for y in (x, odd):
         assert bool(((bias_grad(y).double() - want).abs() <= 2 ** -8 * want.abs() + M * 2 ** -24 * size).all())
+
+
+@pytest.mark.parametrize("rows,H", [(1, 8), (3, 512), (5, 520), (2049, 768), (4100, 1024), (770, 1032)])
+@pytest.mark.parametrize("rms,dres", [(True, True), (True, False), (False, True), (False, False)])
+def test_norm_backward_narrow_rows(rows, H, rms, dres):
+    """A wave per row up to 1024 columns, a block per row above: against float64, ds rounds once (2^-8), dw / db add fp32
+    terms of every row (rows * 2^-24 of their sizes) and round once."""
+    from distributed_llm_alignment_amd.ops import _ext
+
+    g0 = torch.Generator(device=DEV).manual_seed(rows + H)
+
+    def r(*s):
+        return torch.randn(*s, generator=g0, device=DEV).bfloat16()
+
+    s, dy, w, add = r(rows, H), r(rows, H), r(H), (r(rows, H) if dres else None)
+    sd, dyd, wd = s.double(), dy.double(), w.double()
+    mean = torch.zeros(rows, 1, device=DEV, dtype=torch.float64) if rms else sd.mean(1, keepdim=True)
+    rstd = ((sd - mean).pow(2).mean(1, keepdim=True) + 1e-5).rsqrt()
+    ds, dw, db = _ext.require().norm_bwd(dy, s, w, rstd.float().view(-1), None if rms else mean.float().view(-1), add, not rms, rms)
+    xh, g = (sd - mean) * rstd, dyd * wd
+    want = (g - xh * (g * xh).mean(1, keepdim=True) - (0 if rms else g.mean(1, keepdim=True))) * rstd
+    size = want.abs().amax() if want.numel() else 0
+    if dres:
+        want = want + add.double()
+    assert bool(((ds.double() - want).abs() <= 2 ** -8 * want.abs() + 1e-5 * size + 1e-6).all())
+    for have, term in ((dw, dyd * xh), (db, dyd)):
+        if have.numel():
+            t = term.sum(0)
+            assert bool(((have.double() - t).abs() <= 2 ** -8 * t.abs() + (rows + 16) * 2 ** -23 * term.abs().sum(0)).all())
