@@ -44,12 +44,12 @@ def _ref_linear_logprob(hidden, weight, targets):
 
 
 def _logits(hidden: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
-    """hidden @ weight^T with rows that start at multiples of 128 bytes, whatever the vocabulary is: with GPT-2's 50257
-    columns side by side every row starts elsewhere, and the products around the logits (8000 rows, width 768)
-    take 662 / 833 / 768 us (logits, their two gradients) against 544 / 800 / 631 with rows of 50304. Small heads
-    gain nothing on the GPU and pay the calls below on the host."""
+    """hidden @ weight^T, for a vocabulary that is no multiple of 8 with rows that start at multiples of 128 bytes: with
+    GPT-2's 50257 columns side by side every row starts elsewhere, and the products around the logits (8000 rows,
+    width 768) take 662 / 833 / 768 us (logits, their two gradients) against 544 / 800 / 631 with rows of 50304.
+    Small heads gain nothing on the GPU and pay the calls below on the host."""
     V = weight.shape[0]
-    if V % 64 == 0 or V < 8192 or hidden.dtype != torch.bfloat16 or weight.dtype != torch.bfloat16:
+    if V % 8 == 0 or V < 8192 or hidden.dtype != torch.bfloat16 or weight.dtype != torch.bfloat16:
         return F.linear(hidden, weight)
     out = torch.empty((hidden.shape[0], V + -V % 64), dtype=hidden.dtype, device=hidden.device)[:, :V]
     return torch.mm(hidden, weight.t(), out=out)
